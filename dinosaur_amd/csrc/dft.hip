@@ -8,86 +8,47 @@
 // (the algorithmic minimum), versus the reference's dense (I x 2M-1) matmul
 // (spherical_harmonic.py:266-268, 275-276).
 //
-// Other I: a direct real DFT with the cos/sin table in LDS (O(I M) per column).
+// Other I: a mixed-radix FFT when every prime factor is 2, 3, 5 or 7
+// (dft_mixed.hip), else a folded real DFT on the matrix cores up to 513
+// longitudes (dft_gemm.hip).  What remains (longer lengths with a large prime
+// factor, fewer than 8 longitudes): a direct real DFT with the cos/sin table in
+// LDS, O(I M) per column.
 //
 // Real-basis conventions (fourier.py:24-60): row 0 is 1/sqrt(2 pi), row 2m-1
 // is cos(m lambda)/sqrt(pi), row 2m is sin(m lambda)/sqrt(pi).
 #include <algorithm>
 #include <type_traits>
 
-#include "dino_common.h"
+#include "dft_common.h"
 
 namespace dino {
+
+// dft_mixed.hip
+bool dft_mixed_available(int N, bool f64);
+template <typename T>
+int dft_mixed(bool forward, const dino_plan* pl, const T* in, T* out, const T* tw, const T* qw,
+              int64_t B, int weighted, hipStream_t s);
+
+// dft_gemm.hip
+template <typename T>
+int dft_gemm(bool forward, const dino_plan* pl, const T* in, T* out, const T* qw, int64_t B,
+             int weighted, hipStream_t s);
+
+int device_cus() {
+  static int cus[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!cus[dev]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        n <= 0)
+      n = 256;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
+
 namespace {
-
-template <typename T>
-struct cplx {
-  T x, y;
-};
-
-template <typename T>
-__device__ __forceinline__ cplx<T> cadd(cplx<T> a, cplx<T> b) { return {a.x + b.x, a.y + b.y}; }
-template <typename T>
-__device__ __forceinline__ cplx<T> csub(cplx<T> a, cplx<T> b) { return {a.x - b.x, a.y - b.y}; }
-template <typename T>
-__device__ __forceinline__ cplx<T> cmul(cplx<T> a, cplx<T> b) {
-  return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x};
-}
-// multiply by -i (forward) or +i (inverse)
-template <typename T, bool INV>
-__device__ __forceinline__ cplx<T> mul_mi(cplx<T> a) {
-  return INV ? cplx<T>{-a.y, a.x} : cplx<T>{a.y, -a.x};
-}
-
-template <typename T, bool INV>
-__device__ __forceinline__ void dft2(cplx<T>* v) {
-  cplx<T> a = v[0], b = v[1];
-  v[0] = cadd(a, b);
-  v[1] = csub(a, b);
-}
-
-template <typename T, bool INV>
-__device__ __forceinline__ void dft4(cplx<T>& a0, cplx<T>& a1, cplx<T>& a2, cplx<T>& a3) {
-  cplx<T> s02 = cadd(a0, a2), d02 = csub(a0, a2);
-  cplx<T> s13 = cadd(a1, a3), d13 = mul_mi<T, INV>(csub(a1, a3));
-  a0 = cadd(s02, s13);
-  a2 = csub(s02, s13);
-  a1 = cadd(d02, d13);
-  a3 = csub(d02, d13);
-}
-
-template <typename T, bool INV>
-__device__ __forceinline__ void dft4v(cplx<T>* v) { dft4<T, INV>(v[0], v[1], v[2], v[3]); }
-
-template <typename T, bool INV>
-__device__ __forceinline__ void dft8(cplx<T>* v) {
-  const T c = (T)0.70710678118654752440;
-  cplx<T> e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6];
-  cplx<T> o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
-  dft4<T, INV>(e0, e1, e2, e3);
-  dft4<T, INV>(o0, o1, o2, o3);
-  // W8^k for k = 1, 2, 3 (conjugated for the inverse)
-  cplx<T> w1 = INV ? cplx<T>{c, c} : cplx<T>{c, -c};
-  cplx<T> w3 = INV ? cplx<T>{-c, c} : cplx<T>{-c, -c};
-  o1 = cmul(o1, w1);
-  o2 = mul_mi<T, INV>(o2);
-  o3 = cmul(o3, w3);
-  v[0] = cadd(e0, o0);
-  v[4] = csub(e0, o0);
-  v[1] = cadd(e1, o1);
-  v[5] = csub(e1, o1);
-  v[2] = cadd(e2, o2);
-  v[6] = csub(e2, o2);
-  v[3] = cadd(e3, o3);
-  v[7] = csub(e3, o3);
-}
-
-template <typename T, int R, bool INV>
-__device__ __forceinline__ void dft_r(cplx<T>* v) {
-  if constexpr (R == 2) dft2<T, INV>(v);
-  else if constexpr (R == 4) dft4v<T, INV>(v);
-  else dft8<T, INV>(v);
-}
 
 // One in-place Stockham pass on P interleaved complex columns of length N:
 // buf[n * P + p].  All butterflies of the pass are loaded to registers before
@@ -578,20 +539,6 @@ int launch_fft_fixed(bool forward, const dino_plan* pl, const T* in, T* out,
   return DINO_OK;
 }
 
-int device_cus() {
-  static int cus[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cus[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        n <= 0)
-      n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
-}
-
 template <int N>
 int launch_fft_persistent(bool forward, const dino_plan* pl, const float* in, float* out,
                           const float* tw, const float* qw, int64_t B, int weighted,
@@ -663,9 +610,12 @@ int run_dft(bool forward, const dino_plan* pl, const void* in_v, void* out_v, in
       case 512: return launch_fft_n<T, 512>(forward, pl, in, out, tw, qw, B, weighted, s);
       case 1024: return launch_fft_n<T, 1024>(forward, pl, in, out, tw, qw, B, weighted, s);
       case 2048: return launch_fft_n<T, 2048>(forward, pl, in, out, tw, qw, B, weighted, s);
-      default: break;  // 4096 falls through to the direct path
+      default: break;  // 4096: mixed-radix
     }
   }
+  if (pl->dftg32[0]) return dft_gemm<T>(forward, pl, in, out, qw, B, weighted, s);
+  if (dft_mixed_available(pl->I, sizeof(T) == 8))
+    return dft_mixed<T>(forward, pl, in, out, tw, qw, B, weighted, s);
   int N = pl->I;
   int rows = forward ? N : pl->R;
   int TJ = 32;

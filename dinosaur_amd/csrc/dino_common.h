@@ -57,6 +57,10 @@ struct dino_plan {
   float* p32;           // FP32 copy
   double* tw64;         // (I) complex twiddles exp(-2 pi i k / I) as (cos, sin)
   float* tw32;
+  // Coefficients of the longitude transform as a matrix product (dft_gemm.hip),
+  // forward and inverse; null when another kernel serves this length.
+  float* dftg32[2];
+  double* dftg64[2];
   // Forward-transform tables in MFMA fragment order (legendre_rows.hip).
   // fks = number of 32-node reduction steps the tables hold (1, 2, 4 or 8;
   // 0 when Jh > 256 and the tiled kernels are used instead).

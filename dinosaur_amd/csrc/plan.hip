@@ -155,6 +155,10 @@ __global__ void quad_weights_kernel(int I, int J, const double* w, double* q64,
   q32[j] = (float)q;
 }
 
+bool dft_mixed_available(int N, bool f64);
+bool dft_gemm_available(int I, int M);
+int64_t dft_gemm_table_elems(const dino_plan* pl, bool inverse);
+void dft_gemm_table_fill(const dino_plan* pl, hipStream_t s);
 int forward_fragment_steps(int Jh);
 int64_t forward_fragment_layout(int M, int L, int ks, int64_t* off);
 void forward_fragment_fill(const dino_plan* pl, hipStream_t s);
@@ -166,7 +170,8 @@ static void free_plan(dino_plan* p) {
   if (!p) return;
   void* bufs[] = {p->nodes64, p->weights64, p->qw32, p->qw64, p->m_offset,
                   p->p64, p->p32,
-                  p->tw64, p->tw32, p->ftile_off, p->ffrag32, p->ffragbf,
+                  p->tw64, p->tw32, p->dftg32[0], p->dftg32[1], p->dftg64[0], p->dftg64[1],
+                  p->ftile_off, p->ffrag32, p->ffragbf,
                   p->itile_off, p->ifrag32, p->ifragbf, p->sink};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
@@ -268,6 +273,15 @@ extern "C" int dino_plan_create(int M, int L, int I, int J, const double* nodes,
   PLAN_HIP(hipGetLastError());
   twiddle_kernel<<<(I + 255) / 256, 256>>>(I, p->tw64, p->tw32);
   PLAN_HIP(hipGetLastError());
+  if (!p->pow2 && !dft_mixed_available(I, false) && dft_gemm_available(I, M)) {
+    for (int inv = 0; inv < 2; ++inv) {
+      const int64_t n = dft_gemm_table_elems(p, inv);
+      PLAN_HIP(hipMalloc(&p->dftg32[inv], sizeof(float) * n));
+      PLAN_HIP(hipMalloc(&p->dftg64[inv], sizeof(double) * n));
+    }
+    dft_gemm_table_fill(p, 0);
+    PLAN_HIP(hipGetLastError());
+  }
   p->fks = forward_fragment_steps(p->Jh);
   if (p->fks > 0) {
     std::vector<int64_t> foff(M);
