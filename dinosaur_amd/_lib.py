@@ -105,13 +105,19 @@ SIGNATURES = {
     'dino_nodal_hybrid_destroy': (_c_i, [_c_p]),
     'dino_nodal_hybrid_fields': (_c_i64, [_c_p, _c_i64, _c_i]),
     'dino_nodal_hybrid_explicit': (_c_i, [_c_p, _c_p, _c_p, _c_i64, _c_i, _c_p]),
+    'dino_held_suarez_create': (_c_i, [_c_i, _c_i, _c_i] + [_c_dp] * 6 + [_c_d] * 6
+                                + [ctypes.POINTER(_c_p)]),
+    'dino_held_suarez_destroy': (_c_i, [_c_p]),
+    'dino_held_suarez_nodal': (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i, _c_p]),
+    'dino_held_suarez_nodal_adjoint': (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i,
+                                              _c_p]),
     'dino_vregrid_create': (_c_i, [_c_i, _c_i, _c_dp, _c_dp, _c_i, _c_dp, _c_dp,
                                    ctypes.POINTER(_c_p)]),
     'dino_vregrid_destroy': (_c_i, [_c_p]),
     'dino_vregrid_apply': (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i, _c_p]),
 }
 VREGRID_CONSERVATIVE_SIGMA, VREGRID_CONSERVATIVE_PRESSURE, VREGRID_LINEAR_SIGMA = 0, 1, 2
-MODAL_HYBRID = 1
+MODAL_HYBRID, MODAL_FORCED = 1, 2
 
 _lib = None
 _lock = threading.Lock()

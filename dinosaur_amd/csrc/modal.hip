@@ -31,6 +31,7 @@
 struct dino_modal {
   int R, L, K, nt, hum;
   int hybrid;  // DINO_MODAL_HYBRID: prep also emits ln ps, no humidity extras
+  int forced;  // DINO_MODAL_FORCED: prep also emits ln ps, epilogue adds a forcing group
   double radius, gravity;
   // device constant block: il[L], ev[L], mask[L], UP, DN, UP2, DN2 (R*L each),
   // jr[R] (coefficient), pr[R] (partner row, stored as a number)
@@ -74,12 +75,12 @@ struct StateGroups {  // state leaves in one buffer: vort, div, temp, lnps, trac
   int64_t z, d, t, lnps, tr[MAXTR], n;
 };
 struct EpiGroups {  // forward-transform output (fields)
-  int64_t cu, cv, ke, te, ut, vt, lsp, trn[MAXTR], tu[MAXTR], tv[MAXTR], curl, dc, n;
+  int64_t cu, cv, ke, te, ut, vt, lsp, trn[MAXTR], tu[MAXTR], tv[MAXTR], curl, dc, ht, n;
 };
 
-// hybrid: the sigma groups of a dry state plus ln ps itself (LN), which the
-// hybrid nodal kernel needs for the column's surface pressure
-inline PrepGroups prep_groups(int K, int nt, bool moist, int64_t E, bool hybrid = false) {
+// lnps: ln ps itself (LN) as a last group, which the hybrid nodal kernel and the
+// Held-Suarez forcing need for the column's surface pressure
+inline PrepGroups prep_groups(int K, int nt, bool moist, int64_t E, bool lnps = false) {
   PrepGroups g;
   std::memset(&g, 0, sizeof(g));
   int64_t o = 0;
@@ -88,7 +89,7 @@ inline PrepGroups prep_groups(int K, int nt, bool moist, int64_t E, bool hybrid 
   for (int i = 0; i < nt; ++i) g.tr[i] = take(K);
   g.u = take(K); g.v = take(K); g.gx = take(1); g.gy = take(1);
   if (moist) { g.lp = take(1); g.qx = take(K); g.qy = take(K); }
-  if (hybrid) g.ln = take(1);
+  if (lnps) g.ln = take(1);
   g.n = o;
   return g;
 }
@@ -104,7 +105,8 @@ inline StateGroups state_groups(int K, int nt, int64_t E) {
   return g;
 }
 
-inline EpiGroups epi_groups(int K, int nt, bool moist, int64_t E) {
+// forced: a temperature tendency (HT) as a last group
+inline EpiGroups epi_groups(int K, int nt, bool moist, int64_t E, bool forced = false) {
   EpiGroups g;
   std::memset(&g, 0, sizeof(g));
   int64_t o = 0;
@@ -113,13 +115,14 @@ inline EpiGroups epi_groups(int K, int nt, bool moist, int64_t E) {
   g.vt = take(K); g.lsp = take(1);
   for (int i = 0; i < nt; ++i) { g.trn[i] = take(K); g.tu[i] = take(K); g.tv[i] = take(K); }
   if (moist) { g.curl = take(K); g.dc = take(K); }
+  if (forced) g.ht = take(K);
   g.n = o;
   return g;
 }
 
 struct MP {
   int R, L, K, nt, hum;  // hum < 0 also on hybrid levels (no humidity extras)
-  int hybrid;
+  int lnps, forced;  // prep emits ln ps; epilogue adds the forcing group
   int kc, nkc;  // levels per thread and level chunks: (logical) grid row = member * nkc + chunk
   int64_t RL;
   double a, g;
@@ -256,7 +259,7 @@ __global__ __launch_bounds__(256) void prep_kernel(const T* __restrict__ st, T* 
   *(W(out, pg.gx, 1, 0) + pos) = S.dlon(lp) * inva;
   *(W(out, pg.gy, 1, 0) + pos) = S.cldl(lp) * inva;
   if (p.hum >= 0) *(W(out, pg.lp, 1, 0) + pos) = lp[pos] * cst[o.ev + l];
-  if (p.hybrid) *(W(out, pg.ln, 1, 0) + pos) = lp[pos];
+  if (p.lnps) *(W(out, pg.ln, 1, 0) + pos) = lp[pos];
 }
 
 template <typename T>
@@ -306,7 +309,7 @@ __global__ __launch_bounds__(256) void prep_adjoint_kernel(const T* __restrict__
   if (kch != 0) return;  // the single-level field, once per member
   T lb = (-S.dlon(F(gout, pg.gx, 1, 0)) + S.cldl_t(F(gout, pg.gy, 1, 0))) * inva;
   if (p.hum >= 0) lb += cst[o.ev + l] * *(F(gout, pg.lp, 1, 0) + pos);
-  if (p.hybrid) lb += *(F(gout, pg.ln, 1, 0) + pos);
+  if (p.lnps) lb += *(F(gout, pg.ln, 1, 0) + pos);
   *(W(gst, sg.lnps, 1, 0) + pos) = lb;
 }
 
@@ -355,7 +358,8 @@ __global__ __launch_bounds__(256) void epilogue_kernel(const T* __restrict__ in,
     }
     *(W(st, sg.z, K, k) + pos) = vort * mask;
     *(W(st, sg.d, K, k) + pos) = div * mask;
-    *(W(st, sg.t, K, k) + pos) = temp * mask;
+    const T forcing = p.forced ? *(F(in, eg.ht, K, k) + pos) : (T)0;
+    *(W(st, sg.t, K, k) + pos) = temp * mask + forcing;
     for (int i = 0; i < MAXTR; ++i) {
       if (i >= p.nt) break;
       T v = *(F(in, eg.trn[i], K, k) + pos) -
@@ -434,6 +438,7 @@ __global__ __launch_bounds__(256) void epilogue_adjoint_kernel(const T* __restri
       *(W(gin, eg.curl, K, k) + pos) = zm;
       *(W(gin, eg.dc, K, k) + pos) = -dm;
     }
+    if (p.forced) *(W(gin, eg.ht, K, k) + pos) = tb[S.row + l];
   }
   if (kch == 0) *(W(gin, eg.lsp, 1, 0) + pos) = MB(F(gst, sg.lnps, 1, 0));
 }
@@ -451,7 +456,8 @@ MP make_mp(const dino_modal* m) {
   p.K = m->K;
   p.nt = m->nt;
   p.hum = m->hybrid ? -1 : m->hum;
-  p.hybrid = m->hybrid;
+  p.lnps = m->hybrid || m->forced;
+  p.forced = m->forced;
   p.kc = DINO_MODAL_LEVELS_PER_THREAD < m->K ? DINO_MODAL_LEVELS_PER_THREAD : m->K;
   p.nkc = (m->K + p.kc - 1) / p.kc;
   p.RL = (int64_t)m->R * m->L;
@@ -469,7 +475,7 @@ int run(int which, const dino_modal* m, const void* a, const void* b, void* out,
     p.kc *= 2;
     p.nkc = (m->K + p.kc - 1) / p.kc;
   }
-  const bool moist = m->hum >= 0 && !m->hybrid, hyb = m->hybrid != 0;
+  const bool moist = m->hum >= 0 && !m->hybrid, lnps = p.lnps != 0, forced = p.forced != 0;
   StateGroups sg = state_groups(m->K, m->nt, E);
   const unsigned gy = (unsigned)(E * p.nkc);
   dim3 grid((unsigned)((p.RL + 255) / 256), gy);
@@ -478,20 +484,20 @@ int run(int which, const dino_modal* m, const void* a, const void* b, void* out,
   switch (which) {
     case 0:
       prep_kernel<T><<<tgrid, 256, 0, s>>>((const T*)a, (T*)out, c, m->tile_pos, m->n_tile_pos,
-                                           sg, prep_groups(m->K, m->nt, moist, E, hyb), p);
+                                           sg, prep_groups(m->K, m->nt, moist, E, lnps), p);
       break;
     case 1:
       prep_adjoint_kernel<T><<<grid, 256, 0, s>>>((const T*)a, (T*)out, c, sg,
-                                                  prep_groups(m->K, m->nt, moist, E, hyb), p);
+                                                  prep_groups(m->K, m->nt, moist, E, lnps), p);
       break;
     case 2:
       epilogue_kernel<T><<<grid, 256, 0, s>>>((const T*)a, (const T*)b, (T*)out, c,
-                                              epi_groups(m->K, m->nt, moist, E), sg, p);
+                                              epi_groups(m->K, m->nt, moist, E, forced), sg, p);
       break;
     default:
       epilogue_adjoint_kernel<T><<<tgrid, 256, 0, s>>>((const T*)a, (T*)out, c, m->tile_pos,
                                                        m->n_tile_pos,
-                                                       epi_groups(m->K, m->nt, moist, E), sg, p);
+                                                       epi_groups(m->K, m->nt, moist, E, forced), sg, p);
   }
   DINO_LAUNCH_CHECK("modal kernel");
   return DINO_OK;
@@ -508,7 +514,7 @@ extern "C" int dino_modal_create_ex(int R, int L, int K, int n_tracers, int humi
                                     const double* dn, const double* up2, const double* dn2,
                                     int flags, dino_modal** out) {
   DINO_REQUIRE(out, DINO_EINVAL, "dino_modal_create: out is NULL");
-  DINO_REQUIRE((flags & ~DINO_MODAL_HYBRID) == 0, DINO_EINVAL, "unknown modal flags 0x%x",
+  DINO_REQUIRE((flags & ~(DINO_MODAL_HYBRID | DINO_MODAL_FORCED)) == 0, DINO_EINVAL, "unknown modal flags 0x%x",
                flags);
   *out = nullptr;
   DINO_REQUIRE(R >= 1 && R % 2 == 1 && L >= 2 && K >= 1 && (int64_t)R * L < (int64_t)1 << 31,
@@ -556,6 +562,7 @@ extern "C" int dino_modal_create_ex(int R, int L, int K, int n_tracers, int humi
   m->nt = n_tracers;
   m->hum = humidity_index;
   m->hybrid = (flags & DINO_MODAL_HYBRID) ? 1 : 0;
+  m->forced = (flags & DINO_MODAL_FORCED) ? 1 : 0;
   m->radius = radius;
   m->gravity = gravity;
   hipError_t e = hipMalloc(&m->c64, sizeof(double) * o.total);
@@ -600,8 +607,8 @@ extern "C" int64_t dino_modal_fields(const dino_modal* m, int64_t members, int w
   if (!m || members < 0) return -1;
   const bool moist = m->hum >= 0 && !m->hybrid;
   if (which == 0) return state_groups(m->K, m->nt, members).n;
-  if (which == 1) return prep_groups(m->K, m->nt, moist, members, m->hybrid != 0).n;
-  return epi_groups(m->K, m->nt, moist, members).n;
+  if (which == 1) return prep_groups(m->K, m->nt, moist, members, m->hybrid || m->forced).n;
+  return epi_groups(m->K, m->nt, moist, members, m->forced != 0).n;
 }
 
 #define MODAL_ENTRY(NAME, WHICH)                                                            \

@@ -1,11 +1,15 @@
 """Held-Suarez forcing on sigma levels (mirrors dinosaur/held_suarez.py:47-167)."""
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
+from . import _lib
 from . import primitive_equations
 from . import scales
+from . import spherical_harmonic
 from . import time_integration
 
 units = scales.units
@@ -87,3 +91,67 @@ class HeldSuarezForcingSigma(time_integration.ExplicitODE):
         tracers={k: torch.zeros_like(v) for k, v in state.tracers.items()},
         sim_time=None,
     )
+
+  # ---- fused with the primitive equations
+  def handle(self, device):
+    """The forcing's constants on a device, for the nodal kernels."""
+    scalars = [float(x) for x in (self.minT, self.maxT, self.dTy, self.dThz,
+                                  self.physics_specs.kappa, self.p0)]
+    key = (torch.device(device).index, *scalars)
+    cache = self.__dict__.setdefault('_handles', {})
+    h = cache.get(key)
+    if h is None:
+      grid = self.coords.horizontal
+      f64 = lambda a: np.ascontiguousarray(np.asarray(a, np.float64))  # noqa: E731
+      sin2 = np.sin(self.lat[0]) ** 2
+      cos2 = np.cos(self.lat[0]) ** 2
+      arrays = [f64(a) for a in ((self.kv() / grid.cos_lat ** 2)[:, 0], self.kt()[:, 0],
+                                 self.sigma, self.reference_temperature, sin2, cos2)]
+      out = ctypes.c_void_p()
+      with torch.cuda.device(device):
+        rc = _lib.lib().dino_held_suarez_create(
+            len(self.sigma), grid.longitude_nodes, grid.latitude_nodes,
+            *(_lib.dptr(a) for a in arrays), *scalars, ctypes.byref(out))
+      _lib.check(rc, 'dino_held_suarez_create')
+      h = primitive_equations._Handle(out, 'dino_held_suarez_destroy')
+      cache[key] = h
+    return h
+
+  def fused_with(self, equation):
+    """The sum of `equation` and this forcing with the forcing applied between
+    the equation's two transforms, or None when the fused kernels do not serve
+    the pair (another equation class, grid implementation or coordinates, or
+    replaced methods); see time_integration.compose_equations."""
+    eq, pe = type(equation), primitive_equations.PrimitiveEquationsSigma
+    own = (isinstance(equation, pe) and type(self) is HeldSuarezForcingSigma
+           and eq.explicit_terms is pe.explicit_terms
+           and eq._explicit_fused is pe._explicit_fused
+           and not {'explicit_terms', 'equilibrium_temperature'} & set(self.__dict__))
+    if not own or not equation.fused_nodal:
+      return None
+    a, b = self.coords, equation.coords
+    if not (isinstance(b.horizontal.spherical_harmonics,
+                       spherical_harmonic.RealSphericalHarmonics)
+            and a.horizontal == b.horizontal and a.vertical == b.vertical
+            and self.reference_temperature.shape == (b.vertical.layers,)):
+      return None
+    return _ForcedEquations(equation, self)
+
+
+class _ForcedEquations:
+  """Primitive equations with a nodal forcing between their transforms: the
+  explicit terms and the fused IMEX step's hooks."""
+
+  def __init__(self, equation, forcing):
+    self.equation, self.forcing = equation, forcing
+
+  def explicit_terms(self, state):
+    eq = self.equation
+    primitive_equations.validate_state_shape(state, eq.coords)
+    return eq._explicit_fused(state, eq._check_tracers(state), self.forcing)
+
+  def flat_imex_ops(self, state):
+    ops = self.equation._flat_imex_ops(state)
+    if ops is not None:
+      ops.explicit_terms = self.explicit_terms
+    return ops

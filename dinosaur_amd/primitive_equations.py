@@ -498,6 +498,61 @@ class _NodalFused(torch.autograd.Function):
     return gin, None, None
 
 
+class _NodalForced(torch.autograd.Function):
+  """_NodalFused followed by the Held-Suarez forcing on the same buffers: one
+  more input group (ln ps) and one more output group (its temperature
+  tendency)."""
+
+  @staticmethod
+  def forward(ctx, nodal, h, members, forcing, K, nt):
+    nodal = nodal.contiguous()
+    lib = _lib.lib()
+    E = members
+    n_in = lib.dino_nodal_fields(h.handle, E, 0)
+    n_out = lib.dino_nodal_fields(h.handle, E, 1)
+    if nodal.shape[0] != n_in + E:
+      raise ValueError(f'forced nodal kernels expect {n_in + E} input fields, got {nodal.shape[0]}')
+    out = torch.empty((n_out + E * K,) + tuple(nodal.shape[1:]), dtype=nodal.dtype,
+                      device=nodal.device)
+    code = _lib.DINO_F64 if nodal.dtype == torch.float64 else _lib.DINO_F32
+    # first fields of T U V LNPS and of CU CV HT
+    groups = ((ctypes.c_int64 * 4)(2 * E * K, (3 + nt) * E * K, (4 + nt) * E * K, n_in),
+              (ctypes.c_int64 * 3)(0, E * K, n_out))
+    if not _lib.skip_values():  # the backward reads only the saved inputs
+      stream = ctypes.c_void_p(torch.cuda.current_stream(nodal.device).cuda_stream)
+      x, y = ctypes.c_void_p(nodal.data_ptr()), ctypes.c_void_p(out.data_ptr())
+      with torch.cuda.device(nodal.device):
+        _lib.check(lib.dino_nodal_explicit(h.handle, x, y, E, code, stream),
+                   'dino_nodal_explicit')
+        _lib.check(lib.dino_held_suarez_nodal(forcing.handle, x, y, *groups, E, code, stream),
+                   'dino_held_suarez_nodal')
+      field = nodal.element_size() * nodal[0].numel()
+      _lib.tally('nodal', field * (n_in + n_out))
+      _lib.tally('held_suarez', field * E * (8 * K + 1))
+    ctx.save_for_backward(nodal)
+    ctx.h, ctx.forcing, ctx.members, ctx.code, ctx.groups = h, forcing, E, code, groups
+    return out
+
+  @staticmethod
+  def backward(ctx, g):
+    (nodal,) = ctx.saved_tensors
+    g = g.contiguous()
+    gin = torch.empty_like(nodal)
+    stream = ctypes.c_void_p(torch.cuda.current_stream(nodal.device).cuda_stream)
+    lib, E, code = _lib.lib(), ctx.members, ctx.code
+    x, gy, gx = (ctypes.c_void_p(t.data_ptr()) for t in (nodal, g, gin))
+    with torch.cuda.device(nodal.device):
+      _lib.check(lib.dino_nodal_explicit_adjoint(ctx.h.handle, x, gy, gx, E, code, stream),
+                 'dino_nodal_explicit_adjoint')
+      _lib.check(lib.dino_held_suarez_nodal_adjoint(ctx.forcing.handle, x, gy, gx, *ctx.groups, E,
+                                                    code, stream),
+                 'dino_held_suarez_nodal_adjoint')
+    field = g.element_size() * nodal[0].numel()
+    _lib.tally('nodal_adjoint', field * (2 * nodal.shape[0] + g.shape[0]))
+    _lib.tally('held_suarez', field * (2 * nodal.shape[0] + g.shape[0]))
+    return gin, None, None, None, None, None
+
+
 class _Handle:
   """Owns a library object created by dino_*_create."""
 
@@ -633,6 +688,7 @@ class _FlatImexOps:
     self.go = self.ib - self.ib % 4
     self.n = (3 * E * K + E + E * K * len(names)) * self.RL
     self.op = eq._implicit
+    self.explicit_terms = eq.explicit_terms
     # Real layout: the stage kernels skip the all-zero part l < m of each field
     real = isinstance(eq.coords.horizontal.spherical_harmonics,
                       spherical_harmonic.RealSphericalHarmonics)
@@ -650,7 +706,7 @@ class _FlatImexOps:
     return State.from_flat(buf, *self.layout)
 
   def explicit(self, buf):
-    out = self.eq.explicit_terms(self.state(buf))
+    out = self.explicit_terms(self.state(buf))
     fb = out.flat_buffer()
     return fb if fb is not None else to_flat(out).flat_buffer()
 
@@ -820,8 +876,8 @@ class PrimitiveEquationsSigma:
     cache[key] = h
     return h
 
-  def _modal_handle(self, device, names):
-    key = (torch.device(device).index, tuple(names))
+  def _modal_handle(self, device, names, flags=0):
+    key = (torch.device(device).index, tuple(names), flags)
     cache = self.__dict__.setdefault('_modal_handles', {})
     h = cache.get(key)
     if h is not None:
@@ -839,11 +895,11 @@ class PrimitiveEquationsSigma:
     handle = ctypes.c_void_p()
     dp = _lib.dptr
     with torch.cuda.device(device):
-      rc = _lib.lib().dino_modal_create(
+      rc = _lib.lib().dino_modal_create_ex(
           R_, L_, self.coords.vertical.layers, len(names), hum, float(grid.radius),
           float(self.physics_specs.g), dp(il), dp(ev), dp(f64(mask)), *(dp(c) for c in cst),
-          ctypes.byref(handle))
-    _lib.check(rc, 'dino_modal_create')
+          flags, ctypes.byref(handle))
+    _lib.check(rc, 'dino_modal_create_ex')
     h = _Handle(handle, 'dino_modal_destroy')
     cache[key] = h
     return h
@@ -977,16 +1033,18 @@ class PrimitiveEquationsSigma:
       return self._explicit_fused(state, names)
     return self._explicit_unfused(state, names)
 
-  def _explicit_fused(self, state: State, names) -> State:
+  def _explicit_fused(self, state: State, names, forcing=None) -> State:
     """prep kernel -> one inverse transform -> fused nodal kernel -> one
-    forward transform -> epilogue kernel, on flat (fields, R, L) buffers."""
+    forward transform -> epilogue kernel, on flat (fields, R, L) buffers.
+    forcing: a nodal forcing that acts between the transforms (an object with
+    `handle(device)`, see held_suarez), or None."""
     grid = self.coords.horizontal
     sh = grid.spherical_harmonics
     flat = to_flat(state)
     buf = flat.flat_buffer()
     lead, K, _ = flat._flat[1:]
     members = int(np.prod(lead)) if lead else 1
-    mh = self._modal_handle(buf.device, names)
+    mh = self._modal_handle(buf.device, names, _lib.MODAL_FORCED if forcing is not None else 0)
     prep = _ModalPrep.apply(buf, mh, members)
     # the modal buffers between the transforms and the prep / epilogue kernels
     # are read only on the triangle l >= m: written triangle-only
@@ -995,7 +1053,11 @@ class PrimitiveEquationsSigma:
     kw_inv = {'_triangle_only_adjoint': True} if own else {}
     kw_fwd = {'_triangle_only': True} if own else {}
     nodal = sh.inverse_transform(prep, **kw_inv)
-    nout = _NodalFused.apply(nodal, self._nodal_handle(buf.device, names), members)
+    nh = self._nodal_handle(buf.device, names)
+    if forcing is None:
+      nout = _NodalFused.apply(nodal, nh, members)
+    else:
+      nout = _NodalForced.apply(nodal, nh, members, forcing.handle(buf.device), K, len(names))
     mod = sh.transform(nout, **kw_fwd)
     tend = _ModalEpilogue.apply(mod, mh, members, self._orography_modal(buf).contiguous())
     return State.from_flat(tend, lead, K, names,

@@ -92,8 +92,18 @@ def compose_equations(equations: Sequence[Any]) -> ImplicitExplicitODE:
   def explicit_fn(x):
     return _tree_sum([e.explicit_terms(x) for e in equations])
 
-  return ImplicitExplicitODE.from_functions(explicit_fn, main.implicit_terms,
-                                            main.implicit_inverse)
+  out = ImplicitExplicitODE.from_functions(explicit_fn, main.implicit_terms,
+                                           main.implicit_inverse)
+  # One forcing that can act inside the main equation's explicit terms (fused_with):
+  # its IMEX steps then run the fused flat-buffer path.
+  others = [e for e in equations if e is not main]
+  fuse = getattr(others[0], 'fused_with', None) if len(others) == 1 else None
+  if fuse is not None:
+    def flat_imex_ops(state):
+      fused = fuse(main)
+      return None if fused is None else fused.flat_imex_ops(state)
+    out._flat_imex_ops = flat_imex_ops
+  return out
 
 
 @dataclasses.dataclass

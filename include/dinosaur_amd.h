@@ -455,6 +455,13 @@ int dino_modal_epilogue_adjoint(const dino_modal* m, const void* tendency_cot,
  * only through the virtual temperature, :2491-2518), and dino_modal_epilogue
  * reads its output groups, which are those of the dry sigma kernel. */
 enum { DINO_MODAL_HYBRID = 1 };
+
+/* DINO_MODAL_FORCED: a nodal forcing runs between the transforms
+ * (dino_held_suarez_nodal).  dino_modal_prep then also writes ln ps itself, as
+ * its last group, and dino_modal_epilogue reads one more group at the end of
+ * its input, K levels of temperature tendency added without the clip of the
+ * top degree. */
+enum { DINO_MODAL_FORCED = 2 };
 int dino_modal_create_ex(int R, int L, int K, int n_tracers, int humidity_index,
                          double radius, double gravity, const double* inv_lap,
                          const double* lap, const double* clip_mask,
@@ -494,6 +501,32 @@ int64_t dino_nodal_hybrid_fields(const dino_nodal_hybrid* n, int64_t members,
 int dino_nodal_hybrid_explicit(const dino_nodal_hybrid* n,
                                const void* nodal_in, void* nodal_out,
                                int64_t members, int dtype, void* stream);
+
+/* Held-Suarez drag and relaxation (dinosaur/held_suarez.py:99-167) on the nodal
+ * buffers of the explicit terms.  kv_cos2 (kv / cos^2 lat), kt: (K, J) rates;
+ * sigma, tref: K; sin2, cos2 (of latitude): J.
+ * in_groups: first fields of T U V LNPS in the (fields, I, J) input buffer;
+ * out_groups: of CU CV HT in the output buffer.  dino_held_suarez_nodal adds the
+ * drag to CU and CV (which dino_nodal_explicit has written) and writes HT, the
+ * temperature tendency.  The adjoint adds to the cotangents of U, V, T (which
+ * dino_nodal_explicit_adjoint has written) and writes that of LNPS. */
+typedef struct dino_held_suarez dino_held_suarez;
+int dino_held_suarez_create(int K, int I, int J, const double* kv_cos2,
+                            const double* kt, const double* sigma,
+                            const double* tref, const double* sin2,
+                            const double* cos2, double min_t, double max_t,
+                            double dty, double dthz, double kappa, double p0,
+                            dino_held_suarez** out);
+int dino_held_suarez_destroy(dino_held_suarez* h);
+int dino_held_suarez_nodal(const dino_held_suarez* h, const void* nodal_in,
+                           void* nodal_out, const int64_t* in_groups,
+                           const int64_t* out_groups, int64_t members,
+                           int dtype, void* stream);
+int dino_held_suarez_nodal_adjoint(const dino_held_suarez* h,
+                                   const void* nodal_in, const void* out_cot,
+                                   void* in_cot, const int64_t* in_groups,
+                                   const int64_t* out_groups, int64_t members,
+                                   int dtype, void* stream);
 
 /* Vertical regridding of nodal columns from hybrid levels (source: K_s
  * layers with interface coefficients a, b, p = a + b ps) to target levels.
