@@ -62,16 +62,17 @@ struct dino_plan {
   float* dftg32[2];
   double* dftg64[2];
   // Forward-transform tables in MFMA fragment order (legendre_rows.hip).
-  // fks = number of 32-node reduction steps the tables hold (1, 2, 4 or 8;
-  // 0 when Jh > 256 and the tiled kernels are used instead).
+  // fks = number of 32-node reduction steps the tables hold, ceil(Jh / 32);
+  // 0 when Jh > 512 and the tiled kernels are used instead.
   int fks;
   int64_t* ftile_off;   // (M) first tile of each m, in 16-byte units
   float* ffrag32;       // FP32 fragments
   uint16_t* ffragbf;    // BF16 hi/lo fragments
   float* sink;          // (256) store target of out-of-range lanes, never read
   // Inverse-transform tables in MFMA fragment order (legendre_inv_rows.hip).
-  // int_nt = 16-node tiles the tables hold (1, 2, 4 or 8; 0 when Jh > 128).
-  int int_nt;
+  // int_nt = 16-node tiles per node block (1, 2, 4, 6 or 8; 0 when Jh > 512),
+  // int_nb node blocks of int_block nodes.
+  int int_nt, int_nb, int_block;
   int64_t* itile_off;   // (M) first tile of each m, in 16-byte units
   float* ifrag32;       // FP32 fragments
   float* ifragbf;       // BF16 hi/lo fragments (16-byte slots)

@@ -16,7 +16,11 @@
 //   * the Legendre values arrive through a double-buffered LDS tile filled
 //     from a plan table stored in fragment order (inverse_fragments_kernel);
 //   * at the end the up / down halves are staged in LDS and written as whole
-//     contiguous row segments.
+//     contiguous row segments;
+//   * above 128 northern nodes the nodes are split into even blocks, one
+//     workgroup each (TL639, 37 fields: 367 us with the tiled kernel, 228 here,
+//     its table of 330 MB being the largest operand).  Node tiles come in 1, 2,
+//     4, 6 or 8 per block (80 or 90 nodes take 6, not 8).
 //
 // Reduction order inside a 32-degree tile lt .. lt + 31: lane group g =
 // lane / 16 holds the degrees lt + 8 g .. lt + 8 g + 7; class q (d-parity)
@@ -66,11 +70,12 @@ __device__ __forceinline__ float bf16_value(unsigned short h) {
 // per CU to overlap the MFMAs with the loads and stores of other waves (the
 // FP32 register budget of 6 waves per SIMD lets 3 such blocks share a CU;
 // the split path would spill under it).
-template <bool BF, int NT, bool VOUT, int WS>
+// BLK: the nodes are split into blocks (Jh > 128) of int_block nodes, one per z.
+template <bool BF, int NT, bool VOUT, int WS, bool BLK>
 __global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows_kernel(
     const float* __restrict__ modal, float* __restrict__ fourier,
     const float4* __restrict__ itab, const int64_t* __restrict__ itile_off, int B, int L,
-    int J, int Jh, int Rrows, int mpair) {
+    int J, int Jh, int Rrows, int mpair, int block_nodes) {
   static_assert(NT % WS == 0, "the waves of a strip split the node tiles evenly");
   constexpr int NTH = 256 * WS;  // threads
   constexpr int NTW = NT / WS;   // node tiles per wave
@@ -99,7 +104,16 @@ __global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows
   const int g = lane >> 4, c16 = lane & 15;
   const int lt0 = leg_tile_start(m, L);
   const int ntile = inv_tiles_of_m(m, L);
+  // node block z: northern nodes jb .. jb + jn - 1
+  const int jb = BLK ? (int)blockIdx.z * block_nodes : 0;
+  const int jn = BLK && Jh - jb > block_nodes ? block_nodes : Jh - jb;
   const float4* tb = itab + itile_off[m];
+  if constexpr (BLK) tb += (int64_t)blockIdx.z * ntile * TF4;
+  // node tiles this wave multiplies: none for a strip without rows, and not
+  // those beyond the block's nodes (uniform; the barriers are kept)
+  const int nuse = BLK ? __builtin_amdgcn_readfirstlane(
+                             row0 + strip * 16 < nrows ? (jn + 15) / 16 - wh * NTW : 0)
+                       : NTW;
   float* const rs = ring + strip * 16 * kRingPitch;  // this strip's rings
 
   // Line loads of this lane: quad q of row rl of the strip (item = 8 rl + q;
@@ -214,6 +228,7 @@ __global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows
       for (int n = 0; n < NTW; ++n)
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
+          if (BLK && n >= nuse) continue;
           const floatx4 p = buf[((wh * NTW + n) * 2 + q) * 64 + lane];
           const shortx4 ph = __builtin_bit_cast(shortx4, __builtin_shufflevector(p, p, 0, 1));
           const shortx4 pl = __builtin_bit_cast(shortx4, __builtin_shufflevector(p, p, 2, 3));
@@ -226,6 +241,7 @@ __global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows
       for (int n = 0; n < NTW; ++n)
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
+          if (BLK && n >= nuse) continue;
           const floatx4 p = buf[((wh * NTW + n) * 2 + q) * 64 + lane];
 #pragma unroll
           for (int u = 0; u < 4; ++u)
@@ -238,7 +254,8 @@ __global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows
   const int qe = (lt0 - m) & 1;
   __syncthreads();  // every wave is done with the table buffers
   float* os = reinterpret_cast<float*>(lds) + strip * 16 * OPITCH;
-  const int ndn = J - Jh;  // southern nodes (the equator of odd J is northern)
+  // southern nodes of the block: their mirrors, but for the equator of odd J (node 0)
+  const int ndn = (jb == 0 && (J & 1)) ? jn - 1 : jn;
   // the output staging rows belong to one strip: its own wave, or two waves
   auto strip_sync = [&]() {
     if constexpr (WS == 1) wave_lds_sync();
@@ -246,7 +263,7 @@ __global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows
   };
 #pragma unroll
   for (int half = 0; half < 2; ++half) {
-    const int len = half == 0 ? Jh : ndn;
+    const int len = half == 0 ? jn : ndn;
 #pragma unroll
     for (int n = 0; n < NTW; ++n)
 #pragma unroll
@@ -256,16 +273,16 @@ __global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows
         const float a0 = acc[n][0][i], a1 = acc[n][1][i];
         const float e = qe ? a1 : a0, o = qe ? a0 : a1;
         if (half == 0) {
-          if (jj < Jh) os[(4 * g + i) * OPITCH + jj] = e + o;
+          if (jj < jn) os[(4 * g + i) * OPITCH + jj] = e + o;
         } else {
-          const int pos = Jh - 1 - jj;  // position in the southern segment
-          if (jj < Jh && pos < ndn) os[(4 * g + i) * OPITCH + pos] = e - o;
+          const int pos = jn - 1 - jj;  // position in the southern segment
+          if (jj < jn && pos < ndn) os[(4 * g + i) * OPITCH + pos] = e - o;
         }
       }
     strip_sync();
-    const int col0 = half == 0 ? J - Jh : 0;
+    const int col0 = half == 0 ? J - Jh + jb : Jh - jb - jn;
     if constexpr (VOUT) {
-      const int n4 = len / 4;  // J % 8 == 0: both halves hold Jh floats
+      const int n4 = len / 4;  // J % 8 == 0: every half block is a multiple of 4 floats
       for (int idx = lane + 64 * wh; idx < 16 * n4; idx += 64 * WS) {
         const int rl = idx / n4, c = idx - rl * n4;
         const int row = row0 + strip * 16 + rl;
@@ -292,21 +309,24 @@ __global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows
 }
 
 // One thread per (tile, node tile, class, lane) slot of one m (blockIdx.y).
-__global__ void inverse_fragments_kernel(int L, int Jh, int Jhp, int NT,
+__global__ void inverse_fragments_kernel(int L, int Jh, int Jhp, int NT, int NB, int block_nodes,
                                          const double* __restrict__ p64,
                                          const int64_t* __restrict__ m_off,
                                          const int64_t* __restrict__ itile_off,
                                          float* __restrict__ f32, float* __restrict__ fbf) {
   const int m = blockIdx.y;
   const int64_t per_tile = inv_tile_f4(NT);  // slots = float4 per tile
-  const int64_t n = per_tile * inv_tiles_of_m(m, L);
+  const int ntile = inv_tiles_of_m(m, L);
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= n) return;
-  const int tile = (int)(idx / per_tile);
-  const int rem = (int)(idx - tile * per_tile);
+  if (idx >= per_tile * ntile * NB) return;
+  const int slab = (int)(idx / per_tile);  // node block z, degree tile
+  const int z = slab / ntile, tile = slab - z * ntile;
+  const int rem = (int)(idx - slab * per_tile);
   const int nt = rem / 128, q = (rem / 64) % 2, lane = rem % 64;
   const int lt = leg_tile_start(m, L) + kTile * tile;
-  const int gg = lane / 16, jj = 16 * nt + lane % 16;
+  const int gg = lane / 16, jl = 16 * nt + lane % 16;
+  // the node within the block; slots beyond it stay zero
+  const int jj = jl < block_nodes ? z * block_nodes + jl : Jh;
   const int64_t out = (itile_off[m] + idx) * 4;  // floats
   unsigned short h[4], lo[4];
   for (int e = 0; e < 4; ++e) {
@@ -329,18 +349,27 @@ __global__ void inverse_fragments_kernel(int L, int Jh, int Jhp, int NT,
 template <bool BF, int NT>
 int launch_inv_rows(const dino_plan* pl, const float* in, float* out, int64_t B, hipStream_t s) {
   const bool vout = pl->J % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-  const dim3 grid((unsigned)((2 * B + kRows - 1) / kRows), (unsigned)pl->M);
+  const dim3 grid((unsigned)((2 * B + kRows - 1) / kRows), (unsigned)pl->M, (unsigned)pl->int_nb);
   const float4* tab = BF ? reinterpret_cast<const float4*>(pl->ifragbf)
                          : reinterpret_cast<const float4*>(pl->ifrag32);
   const int mpair = (pl->sched[DINO_STAGE_LEGENDRE_INVERSE] & DINO_SCHED_MPAIRED) ? 1 : 0;
   // two waves per strip whenever the node tiles split evenly
   constexpr int WS = NT % 2 == 0 ? 2 : 1;
-  if (vout)
-    leg_inv_rows_kernel<BF, NT, true, WS><<<grid, 256 * WS, 0, s>>>(
-        in, out, tab, pl->itile_off, (int)B, pl->L, pl->J, pl->Jh, pl->R, mpair);
-  else
-    leg_inv_rows_kernel<BF, NT, false, WS><<<grid, 256 * WS, 0, s>>>(
-        in, out, tab, pl->itile_off, (int)B, pl->L, pl->J, pl->Jh, pl->R, mpair);
+#define INV_LAUNCH(VO, BK)                                                             \
+  leg_inv_rows_kernel<BF, NT, VO, WS, BK><<<grid, 256 * WS, 0, s>>>(                    \
+      in, out, tab, pl->itile_off, (int)B, pl->L, pl->J, pl->Jh, pl->R, mpair, pl->int_block)
+  // blocks of at least 65 nodes: only the 6- and 8-tile forms
+  if constexpr (NT >= 6) {
+    if (pl->int_nb > 1) {
+      if (vout) INV_LAUNCH(true, true);
+      else INV_LAUNCH(false, true);
+      DINO_LAUNCH_CHECK("legendre inverse rows kernel");
+      return DINO_OK;
+    }
+  }
+  if (vout) INV_LAUNCH(true, false);
+  else INV_LAUNCH(false, false);
+#undef INV_LAUNCH
   DINO_LAUNCH_CHECK("legendre inverse rows kernel");
   return DINO_OK;
 }
@@ -351,6 +380,7 @@ int inv_rows_by_nt(const dino_plan* pl, const float* in, float* out, int64_t B, 
     case 1: return launch_inv_rows<BF, 1>(pl, in, out, B, s);
     case 2: return launch_inv_rows<BF, 2>(pl, in, out, B, s);
     case 4: return launch_inv_rows<BF, 4>(pl, in, out, B, s);
+    case 6: return launch_inv_rows<BF, 6>(pl, in, out, B, s);
     case 8: return launch_inv_rows<BF, 8>(pl, in, out, B, s);
     default:
       set_error("inverse fragment tables hold %d node tiles", pl->int_nt);
@@ -360,28 +390,34 @@ int inv_rows_by_nt(const dino_plan* pl, const float* in, float* out, int64_t B, 
 
 }  // namespace
 
-// Node tiles of 16 the inverse tables use (1, 2, 4 or 8; 0 when Jh > 128 and
-// the tiled kernels are used instead).
-int inverse_fragment_tiles(int Jh) {
-  int nt = 1;
-  while (16 * nt < Jh) nt *= 2;
-  return nt <= 8 ? nt : 0;
+// Node blocks of the inverse tables: nodes per block (a multiple of 16, at most
+// 128, whose accumulators the registers hold) and the node tiles of 16 a block has room
+// for (1, 2, 4, 6 or 8).  Larger grids split evenly: a workgroup per block
+// re-reads the modal rows, which stay in the caches, and reads its own part of
+// the table.  *tiles = 0 beyond 512 nodes (tiled kernels).
+int inverse_fragment_blocks(int Jh, int* tiles, int* block_nodes) {
+  const int nt = (Jh + 15) / 16;
+  const int nb = (nt + 7) / 8;
+  const int tb = (nt + nb - 1) / nb;
+  *block_nodes = 16 * tb;
+  *tiles = Jh > 512 ? 0 : tb <= 2 ? tb : (tb + 1) / 2 * 2;
+  return nb;
 }
 
-int64_t inverse_fragment_layout(int M, int L, int nt, int64_t* off) {
+int64_t inverse_fragment_layout(int M, int L, int nt, int nb, int64_t* off) {
   int64_t acc = 0;
   for (int m = 0; m < M; ++m) {
     off[m] = acc;
-    acc += (int64_t)inv_tiles_of_m(m, L) * inv_tile_f4(nt);
+    acc += (int64_t)inv_tiles_of_m(m, L) * nb * inv_tile_f4(nt);
   }
   return acc;
 }
 
 void inverse_fragment_fill(const dino_plan* pl, hipStream_t s) {
-  const int64_t most = (int64_t)inv_tile_f4(pl->int_nt) * inv_tiles_of_m(0, pl->L);
+  const int64_t most = (int64_t)inv_tile_f4(pl->int_nt) * pl->int_nb * inv_tiles_of_m(0, pl->L);
   const dim3 grid((unsigned)((most + 255) / 256), (unsigned)pl->M);
-  inverse_fragments_kernel<<<grid, 256, 0, s>>>(pl->L, pl->Jh, pl->Jhp, pl->int_nt, pl->p64,
-                                                pl->m_offset, pl->itile_off, pl->ifrag32,
+  inverse_fragments_kernel<<<grid, 256, 0, s>>>(pl->L, pl->Jh, pl->Jhp, pl->int_nt, pl->int_nb,
+                                                pl->int_block, pl->p64, pl->m_offset, pl->itile_off, pl->ifrag32,
                                                 pl->ifragbf);
 }
 

@@ -380,7 +380,7 @@ int legendre_forward_mfma(const dino_plan* pl, const void* fourier, void* modal,
   const int fam = pl->sched[DINO_STAGE_LEGENDRE_FORWARD] & 0xff;
   if (pl->fks > 0 &&
       (fam == DINO_SCHED_AUTO || fam == DINO_SCHED_ROWS || fam == DINO_SCHED_ROWS_WIDE) &&
-      (precision == DINO_PREC_NATIVE || precision == DINO_PREC_BF16X3))
+      (precision == DINO_PREC_NATIVE || (precision == DINO_PREC_BF16X3 && pl->ffragbf)))
     return legendre_forward_rows(pl, in, out, B, precision == DINO_PREC_BF16X3, triangle_only,
                                  fam == DINO_SCHED_ROWS_WIDE, s);
   DINO_REQUIRE((2 * B + TR - 1) / TR <= 65535, DINO_EINVAL, "batch too large");

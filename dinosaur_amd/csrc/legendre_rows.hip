@@ -179,20 +179,20 @@ __global__ __launch_bounds__(64 * NW, (fwd_waves_per_simd<NW, KS>())) void leg_f
   const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
   float4 x0[KT], x1[KT];
   if constexpr (VIN) {
-    // Coalesced loads: lane = (row rho of the wave's strip, 4-node chunk c)
-    // with CPR chunks per half row (the whole reduction width) and RPI rows
-    // per instruction, both compile-time, so no index division; northern
-    // half ascending, its mirror image descending.  Chunks past Jh / 4 and
-    // rows past the batch read a clamped in-range address and are zeroed by
-    // selects, so the loads issue back to back without branches.
-    constexpr int CPR = 8 * KS, RPI = 64 / CPR;
-    static_assert(KT * RPI == 16, "KT load instructions cover the wave's 16 rows");
+    // Coalesced loads: item 64 it + lane = (row rho of the wave's strip,
+    // 4-node chunk c) with CPR chunks per half row (the whole reduction
+    // width), so KT instructions cover the wave's 16 rows without index
+    // division by a runtime value; northern half ascending, its mirror image
+    // descending.  Chunks past Jh / 4 and rows past the batch read a clamped
+    // in-range address and are zeroed by selects, so the loads issue back to
+    // back without branches.
+    constexpr int CPR = 8 * KS;
     const int H4 = Jh / 4;
-    const int c = lane % CPR, cc = c < H4 ? c : H4 - 1;
     floatx4 u[KT], d[KT];
 #pragma unroll
     for (int it = 0; it < KT; ++it) {
-      const int row = row0 + wave * 16 + lane / CPR + RPI * it;
+      const int c = (64 * it + lane) % CPR, cc = c < H4 ? c : H4 - 1;
+      const int row = row0 + wave * 16 + (64 * it + lane) / CPR;
       const bool ok = c < H4 && row < nrows;
       int b, r;
       row_field(m, row < nrows ? row : nrows - 1, &b, &r);
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(64 * NW, (fwd_waves_per_simd<NW, KS>())) void leg_f
       const float sp = pass == 0 ? sgn : -sgn;
 #pragma unroll
       for (int it = 0; it < KT; ++it) {
-        const int rho = lane / CPR + RPI * it;
+        const int rho = (64 * it + lane) / CPR, c = (64 * it + lane) % CPR;
         *reinterpret_cast<floatx4*>(stg + (wave * 16 + rho) * PITCH + 4 * c) = u[it] + sp * d[it];
       }
       wave_lds_sync();  // each wave stages only its own 16 rows
@@ -405,6 +405,179 @@ __global__ __launch_bounds__(64 * NW, (fwd_waves_per_simd<NW, KS>())) void leg_f
   }
 }
 
+// The same contraction for 129 to 512 northern nodes (FP32): two waves share a
+// 16-row strip, each holding the folded rows of one parity (4 KT registers
+// instead of 8 KT, which at 160 nodes left one wave per SIMD and beyond 256
+// did not fit), and both fill the strip's output ring.  NS strips (16 NS rows)
+// per workgroup: the table of a large grid (262 MB at TL639) is the largest
+// operand at common batches, so a workgroup takes as many rows of one m as
+// there are, up to 128.  kt of the KT node groups are in use.
+// TL639, 37 fields: 519 us with the tiled kernel, 223 us here (table and rows
+// 0.08 ms at the copy rate, 10.6 GFLOP of tiles 0.07 ms).
+template <int KT, int NS, bool VIN>
+__global__ __launch_bounds__(128 * NS) void leg_fwd_split_rows_kernel(
+    const float* __restrict__ fourier, float* __restrict__ modal,
+    const float4* __restrict__ ftab, const int64_t* __restrict__ ftile_off,
+    float* __restrict__ sink, int B, int L, int J, int Jh, int Rrows, int ks, int mpair,
+    int skip_zero) {
+  constexpr int NTH = 128 * NS, RPB = 16 * NS;
+  constexpr int PER = (128 * KT + NTH - 1) / NTH;
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  floatx4* const lds = reinterpret_cast<floatx4*>(smem_raw);
+  const int tf4 = tile_f4(ks), kt = 2 * ks;
+  const int m = m_of_block(blockIdx.y, gridDim.y, mpair);
+  const int nrows = (m == 0) ? B : 2 * B;
+  const int row0 = blockIdx.x * RPB;
+  if (row0 >= nrows) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int strip = wave >> 1, par = wave & 1;  // the wave's strip and fold parity
+  const int g = lane >> 4, c16 = lane & 15;
+  const int strip0 = row0 + strip * 16;
+  const bool used = strip0 < nrows;  // a strip without rows only keeps the barriers
+  const int lt0 = leg_tile_start(m, L);
+  const int ntile = tiles_of_m(m, L);
+  const float4* tb = ftab + ftile_off[m];
+
+  floatx4 st[PER];
+  auto load_table = [&](int t) {
+    const float4* src = tb + (int64_t)t * tf4;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int idx = tid + NTH * i;
+      st[i] = ld4(src + (idx < tf4 ? idx : 0));
+    }
+  };
+  load_table(0);
+
+  // Folded rows of this parity in A-operand order: up + d * down, d = +-1.
+  const float sgn = (((lt0 - m) & 1) != 0) == (par != 0) ? 1.f : -1.f;
+  const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+  floatx4 x[KT];
+  {
+    const int row = strip0 + c16;
+    const bool rok = row < nrows;
+    int b, r;
+    row_field(m, rok ? row : nrows - 1, &b, &r);
+    const float* const f = fourier + ((int64_t)b * Rrows + r) * J;
+    const int j0 = 4 * g < Jh ? 4 * g : 0;
+    const float *const up = f + J - Jh + j0, *const down = f + Jh - 4 - j0;
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      const int jj = 16 * t + 4 * g;
+      x[t] = zero;
+      if (16 * t >= Jh) continue;
+      if constexpr (VIN) {
+        // whole groups at constant offsets from two row pointers; the last one
+        // may be partial (Jh % 4 == 0: whole vectors)
+        const bool in = 16 * t + 16 <= Jh || jj < Jh;
+        const int off = in ? 16 * t : 0;
+        const floatx4 u = *reinterpret_cast<const floatx4*>(up + off);
+        const floatx4 dr = *reinterpret_cast<const floatx4*>(down - off);
+        const floatx4 v = u + sgn * floatx4{dr[3], dr[2], dr[1], dr[0]};
+        x[t] = rok && in ? v : zero;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int q = jj + e;
+          const bool ok = rok && q < Jh;
+          // odd J: node 0 is the equator, counted once
+          const bool okd = ok && !((J & 1) && q == 0);
+          const float uu = f[ok ? J - Jh + q : 0];
+          const float dd = f[okd ? Jh - 1 - q : 0];
+          x[t][e] = (ok ? uu : 0.f) + sgn * (okd ? dd : 0.f);
+        }
+      }
+    }
+  }
+  if (par == 0) zero_block(modal, m, strip0, nrows, Rrows, L, lt0, lane, skip_zero);
+
+  // Output in whole 128-byte lines from a two-tile ring, as in
+  // leg_fwd_rows_kernel; wave `par` stores rows 8 par + lane / 8 of the strip.
+  float* const obase = modal + (int64_t)(m == 0 ? row0 : row0 >> 1) * Rrows * L;
+  auto row_offset = [&](int rl) -> int {
+    const int row = strip0 + rl;
+    if (row >= nrows) return -1;
+    int b, r;
+    row_field(m, row, &b, &r);
+    return ((b - (m == 0 ? row0 : row0 >> 1)) * Rrows + r) * L;
+  };
+  auto ring_origin = [&](int off) -> int {
+    return off < 0 ? 0 : (int)((reinterpret_cast<uintptr_t>(obase + off) >> 2) & 63);
+  };
+  const int rl = 8 * par + (lane >> 3);
+  const int orow = row_offset(rl);
+  const int ra_s = ring_origin(orow);
+  int hi = L;
+  if (orow >= 0) {
+    int b, r;
+    row_field(m, strip0 + rl, &b, &r);
+    hi = L + next_row_head(obase + orow + L, r, Rrows, L);
+  }
+  int ra_w[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) ra_w[i] = ring_origin(row_offset(4 * g + i));
+  float* const rg = reinterpret_cast<float*>(lds + 2 * tf4) + strip * 16 * kRingPitch;
+  if (par == 0)
+    for (int i = lane; i < 16 * kRingPitch / 4; i += 64) reinterpret_cast<floatx4*>(rg)[i] = zero;
+
+  for (int tt = 0; tt < ntile; ++tt) {
+    floatx4* buf = lds + (tt & 1) * tf4;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int idx = tid + NTH * i;
+      if (idx < tf4) buf[idx] = st[i];
+    }
+    // also orders the ring's zeros and the previous tile's ring reads before
+    // this tile's ring writes
+    __syncthreads();
+    // the last iteration reloads its own tile, which is never stored
+    load_table(tt + 1 < ntile ? tt + 1 : tt);
+    __builtin_amdgcn_sched_barrier(0);
+    const int lt = lt0 + tt * kTileDeg;
+    if (used) {
+      // two accumulator chains (even and odd groups), so that the matrix core
+      // need not wait for the previous product
+      floatx4 a0 = zero, a1 = zero;
+#pragma unroll
+      for (int t = 0; t < KT; t += 2) {
+        if (t >= kt) continue;  // kt is even
+        // reads a tile's table a few groups ahead, not all of it (registers)
+        if (t % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+        const floatx4 p0 = buf[(par * kt + t) * 64 + lane];
+        const floatx4 p1 = buf[(par * kt + t + 1) * 64 + lane];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[t][u], p0[u], a0, 0, 0, 0);
+          a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[t + 1][u], p1[u], a1, 0, 0, 0);
+        }
+      }
+      // degrees lt + 2 c16 + par of rows 4 g + i
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        rg[(4 * g + i) * kRingPitch + ((ra_w[i] + lt + 2 * c16 + par) & 63)] = a0[i] + a1[i];
+    }
+    __syncthreads();  // both parities are in the ring
+    const int nk = tt + 1 < ntile ? 1 : 2;
+    for (int k = 0; k < nk; ++k) {
+      const int l4 = lt - ((ra_s + lt0) & 31) + 32 * k + 4 * (lane & 7);
+      const floatx4 v = *reinterpret_cast<const floatx4*>(rg + rl * kRingPitch + ((ra_s + l4) & 63));
+      floatx4 w;  // degrees >= L: the next row's zero head
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = l4 + e < L ? v[e] : 0.f;
+      const bool rok = orow >= 0;
+      const bool full = rok && l4 >= 0 && l4 + 3 < hi;
+      floatx4* const dst = full ? reinterpret_cast<floatx4*>(obase + orow + l4)
+                                : reinterpret_cast<floatx4*>(sink) + lane;
+      *dst = w;
+      if (rok && !full && l4 + 3 >= 0 && l4 < hi) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (l4 + e >= 0 && l4 + e < hi) obase[orow + l4 + e] = w[e];
+      }
+    }
+  }
+}
+
 // One thread per fragment slot of every tile of one m (blockIdx.y = m).
 // FP32 slot order [tile][q][t][lane][e]; BF16 [tile][q][s][h][lane][e'].
 __global__ void forward_fragments_kernel(int L, int Jh, int Jhp, int ks,
@@ -444,8 +617,10 @@ __global__ void forward_fragments_kernel(int L, int Jh, int Jhp, int ks,
     const __bf16 lo = (__bf16)(float)(v - (double)(float)hi);
     const int64_t ub = base * 2;  // uint16 units
     const int64_t pos = ((int64_t)(q * ks + s) * 2) * 512 + lane * 8 + e;
-    fbf[ub + pos] = __builtin_bit_cast(uint16_t, hi);
-    fbf[ub + pos + 512] = __builtin_bit_cast(uint16_t, lo);
+    if (fbf) {
+      fbf[ub + pos] = __builtin_bit_cast(uint16_t, hi);
+      fbf[ub + pos + 512] = __builtin_bit_cast(uint16_t, lo);
+    }
   }
 }
 
@@ -475,23 +650,71 @@ int rows_by_ks(const dino_plan* pl, const float* in, float* out, int64_t B, int 
   switch (pl->fks) {
     case 1: return launch_rows<BF, 1, NW>(pl, in, out, B, skip_zero, s);
     case 2: return launch_rows<BF, 2, NW>(pl, in, out, B, skip_zero, s);
+    case 3: return launch_rows<BF, 3, NW>(pl, in, out, B, skip_zero, s);
     case 4: return launch_rows<BF, 4, NW>(pl, in, out, B, skip_zero, s);
-    case 8: return launch_rows<BF, 8, NW>(pl, in, out, B, skip_zero, s);
-    default:
-      set_error("forward fragment tables hold %d steps", pl->fks);
-      return DINO_EINVAL;
+    default: break;
   }
+  if constexpr (BF && NW == 4) {
+    switch (pl->fks) {
+      case 5: return launch_rows<BF, 5, NW>(pl, in, out, B, skip_zero, s);
+      case 6: return launch_rows<BF, 6, NW>(pl, in, out, B, skip_zero, s);
+      case 7: return launch_rows<BF, 7, NW>(pl, in, out, B, skip_zero, s);
+      case 8: return launch_rows<BF, 8, NW>(pl, in, out, B, skip_zero, s);
+      default: break;
+    }
+  }
+  set_error("forward fragment tables hold %d steps", pl->fks);
+  return DINO_EINVAL;
+}
+
+template <int KT, int NS>
+int launch_split_rows(const dino_plan* pl, const float* in, float* out, int64_t B, int skip_zero,
+                      hipStream_t s) {
+  const bool vin = pl->J % 8 == 0 && reinterpret_cast<uintptr_t>(in) % 16 == 0;
+  const dim3 grid((unsigned)((2 * B + 16 * NS - 1) / (16 * NS)), (unsigned)pl->M);
+  const int mpair = (pl->sched[DINO_STAGE_LEGENDRE_FORWARD] & DINO_SCHED_MPAIRED) ? 1 : 0;
+  const size_t lds = 16 * (size_t)(2 * tile_f4(pl->fks)) + 4 * (size_t)(16 * NS * kRingPitch);
+  const float4* tab = reinterpret_cast<const float4*>(pl->ffrag32);
+#define SPLIT_LAUNCH(VI)                                                                      \
+  do {                                                                                        \
+    const void* k = (const void*)leg_fwd_split_rows_kernel<KT, NS, VI>;                       \
+    DINO_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));   \
+    leg_fwd_split_rows_kernel<KT, NS, VI><<<grid, 128 * NS, lds, s>>>(                         \
+        in, out, tab, pl->ftile_off, pl->sink, (int)B, pl->L, pl->J, pl->Jh, pl->R, pl->fks,  \
+        mpair, skip_zero);                                                                    \
+  } while (0)
+  if (vin) SPLIT_LAUNCH(true);
+  else SPLIT_LAUNCH(false);
+#undef SPLIT_LAUNCH
+  DINO_LAUNCH_CHECK("legendre forward split rows kernel");
+  return DINO_OK;
+}
+
+// Two node groups per 32-node step; 128-row workgroups (16 waves) up to 320
+// nodes, whose fragments fit the 128 registers that 16 waves leave each.
+int split_rows_by_ks(const dino_plan* pl, const float* in, float* out, int64_t B, int skip_zero,
+                     hipStream_t s) {
+  const bool few = 2 * B <= 64;  // rows of one m fit 64-row workgroups
+  if (pl->fks <= 6)
+    return few ? launch_split_rows<12, 4>(pl, in, out, B, skip_zero, s)
+               : launch_split_rows<12, 8>(pl, in, out, B, skip_zero, s);
+  if (pl->fks <= 10)
+    return few ? launch_split_rows<20, 4>(pl, in, out, B, skip_zero, s)
+               : launch_split_rows<20, 8>(pl, in, out, B, skip_zero, s);
+  return launch_split_rows<32, 4>(pl, in, out, B, skip_zero, s);
 }
 
 }  // namespace
 
-// Number of 32-node steps the fragment tables use for this plan (a power of
-// two covering Jh), or 0 when Jh is too large for register-resident rows.
+// Number of 32-node steps the fragment tables use for this plan, or 0 when Jh
+// is too large for register-resident rows.
 int forward_fragment_steps(int Jh) {
-  int ks = 1;
-  while (32 * ks < Jh) ks *= 2;
-  return ks <= 8 ? ks : 0;
+  const int ks = (Jh + 31) / 32;
+  return ks <= 16 ? ks : 0;
 }
+
+// Whether the split-BF16 row kernels serve a table of ks steps.
+bool forward_split_available(int ks) { return ks >= 1 && ks <= 8; }
 
 // Float4 units of the fragment tables; fills off[m] (float4 units).
 int64_t forward_fragment_layout(int M, int L, int ks, int64_t* off) {
@@ -511,8 +734,6 @@ void forward_fragment_fill(const dino_plan* pl, hipStream_t s) {
                                                 pl->ffragbf);
 }
 
-bool forward_rows_available(const dino_plan* pl) { return pl->fks > 0; }
-
 int legendre_forward_rows(const dino_plan* pl, const float* in, float* out, int64_t B,
                           bool split, bool triangle_only, bool wide, hipStream_t s) {
   if (B == 0) return DINO_OK;
@@ -521,7 +742,8 @@ int legendre_forward_rows(const dino_plan* pl, const float* in, float* out, int6
   DINO_REQUIRE((int64_t)8 * kRowsPerWave * pl->R * pl->L < (int64_t)1 << 31, DINO_EINVAL,
                "modal fields too large for the row kernel");
   const int z = triangle_only ? 1 : 0;
-  if (wide)
+  if (!split && pl->fks > 4) return split_rows_by_ks(pl, in, out, B, z, s);
+  if (wide && pl->fks <= 4)
     return split ? rows_by_ks<true, 8>(pl, in, out, B, z, s)
                  : rows_by_ks<false, 8>(pl, in, out, B, z, s);
   return split ? rows_by_ks<true, 4>(pl, in, out, B, z, s)

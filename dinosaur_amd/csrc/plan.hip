@@ -160,10 +160,11 @@ bool dft_gemm_available(int I, int M);
 int64_t dft_gemm_table_elems(const dino_plan* pl, bool inverse);
 void dft_gemm_table_fill(const dino_plan* pl, hipStream_t s);
 int forward_fragment_steps(int Jh);
+bool forward_split_available(int ks);
 int64_t forward_fragment_layout(int M, int L, int ks, int64_t* off);
 void forward_fragment_fill(const dino_plan* pl, hipStream_t s);
-int inverse_fragment_tiles(int Jh);
-int64_t inverse_fragment_layout(int M, int L, int nt, int64_t* off);
+int inverse_fragment_blocks(int Jh, int* tiles, int* block_nodes);
+int64_t inverse_fragment_layout(int M, int L, int nt, int nb, int64_t* off);
 void inverse_fragment_fill(const dino_plan* pl, hipStream_t s);
 
 static void free_plan(dino_plan* p) {
@@ -288,16 +289,16 @@ extern "C" int dino_plan_create(int M, int L, int I, int J, const double* nodes,
     const int64_t f4 = forward_fragment_layout(M, L, p->fks, foff.data());
     PLAN_HIP(hipMalloc(&p->ftile_off, sizeof(int64_t) * M));
     PLAN_HIP(hipMalloc(&p->ffrag32, 16 * f4));
-    PLAN_HIP(hipMalloc(&p->ffragbf, 16 * f4));
+    if (forward_split_available(p->fks)) PLAN_HIP(hipMalloc(&p->ffragbf, 16 * f4));
     PLAN_HIP(hipMalloc(&p->sink, sizeof(float) * 256));
     PLAN_HIP(hipMemcpy(p->ftile_off, foff.data(), sizeof(int64_t) * M, hipMemcpyHostToDevice));
     forward_fragment_fill(p, 0);
     PLAN_HIP(hipGetLastError());
   }
-  p->int_nt = inverse_fragment_tiles(p->Jh);
+  p->int_nb = inverse_fragment_blocks(p->Jh, &p->int_nt, &p->int_block);
   if (p->int_nt > 0) {
     std::vector<int64_t> ioff(M);
-    const int64_t f4 = inverse_fragment_layout(M, L, p->int_nt, ioff.data());
+    const int64_t f4 = inverse_fragment_layout(M, L, p->int_nt, p->int_nb, ioff.data());
     PLAN_HIP(hipMalloc(&p->itile_off, sizeof(int64_t) * M));
     PLAN_HIP(hipMalloc(&p->ifrag32, 16 * f4));
     PLAN_HIP(hipMalloc(&p->ifragbf, 16 * f4));
