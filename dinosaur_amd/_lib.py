@@ -26,6 +26,8 @@ SCHED_MPAIRED = 0x100
 TARGET_ACCUMULATE, TARGET_IDENTITY, TARGET_RANGED = 1, 2, 4
 GATHER_IDENTITY, GATHER_SCALED, GATHER_IMPLICIT_RANGE = 1, 2, 4
 SHT_TRIANGLE_ONLY = 0x100
+SHT_SEC_LAT = 0x200
+WINDS_FROM_VOR_DIV, WINDS_TO_VOR_DIV = 0, 2  # + 1: the adjoint
 STAGE_TRIANGLE_ONLY = 0x100  # dtype flag of dino_imex_stage_ranged[_scaled]
 PRECISIONS = {'native': PREC_NATIVE, 'float32': PREC_NATIVE, 'float64': PREC_NATIVE,
               'bf16x3': PREC_BF16X3}
@@ -97,6 +99,7 @@ SIGNATURES = {
     'dino_modal_prep_adjoint': (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i, _c_p]),
     'dino_modal_epilogue': (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i, _c_p]),
     'dino_modal_epilogue_adjoint': (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_i64, _c_i, _c_p]),
+    'dino_modal_winds': (_c_i, [_c_p, _c_i, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i, _c_i, _c_p]),
     'dino_modal_create_ex': (_c_i, [_c_i, _c_i, _c_i, _c_i, _c_i, _c_d, _c_d, _c_dp, _c_dp, _c_dp,
                                     _c_dp, _c_dp, _c_dp, _c_dp, _c_i, ctypes.POINTER(_c_p)]),
     'dino_nodal_hybrid_create': (_c_i, [_c_i, _c_i, _c_i, _c_i, _c_i, ctypes.POINTER(_c_i), _c_i,

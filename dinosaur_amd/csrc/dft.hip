@@ -589,12 +589,14 @@ int run_dft(bool forward, const dino_plan* pl, const void* in_v, void* out_v, in
   T* out = static_cast<T*>(out_v);
   const T* tw;
   const T* qw;
+  // weights by code: 1 quadrature, 2 1 / cos(lat), 3 both
+  const int wrow = weighted > 0 ? weighted - 1 : 0;
   if constexpr (sizeof(T) == 8) {
     tw = pl->tw64;
-    qw = pl->qw64;
+    qw = pl->qw64 + wrow * (int64_t)pl->qw_stride;
   } else {
     tw = pl->tw32;
-    qw = pl->qw32;
+    qw = pl->qw32 + wrow * (int64_t)pl->qw_stride;
   }
   if (B == 0) return DINO_OK;
   DINO_REQUIRE(B <= 65535, DINO_EINVAL, "batch %lld exceeds 65535 fields per call",

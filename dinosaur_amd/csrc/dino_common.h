@@ -50,8 +50,10 @@ struct dino_plan {
   // device arrays
   double* nodes64;      // (J) ascending
   double* weights64;    // (J) Gauss weights (sum 2)
-  float* qw32;          // (J) (2 pi / I) * w_j
+  // latitude weights (3, qw_stride): (2 pi / I) w_j, 1 / cos(lat_j), their product
+  float* qw32;
   double* qw64;
+  int qw_stride;        // J padded to a multiple of 4: every row starts aligned
   int64_t* m_offset;    // (M) start of row l = m of each m block in the table
   double* p64;          // folded table, FP64
   float* p32;           // FP32 copy

@@ -443,6 +443,65 @@ __global__ __launch_bounds__(256) void epilogue_adjoint_kernel(const T* __restri
   if (kch == 0) *(W(gin, eg.lsp, 1, 0) + pos) = MB(F(gst, sg.lnps, 1, 0));
 }
 
+// ---------------------------------------------------------------- winds
+// Vorticity and divergence <-> cos(lat)-weighted winds (spherical_harmonic.py:
+// 1164-1210), each direction and its adjoint, on pairs of (B, R, L) buffers:
+//   0: (vorticity, divergence) -> (u cos, v cos), read by the inverse transform
+//   1: its adjoint             2: (u, v) / cos -> (vorticity, divergence)
+//   3: its adjoint, read by the inverse transform
+// One pass over both fields instead of about 20 elementwise tensor operations
+// of the composed operators; bound by launches at common sizes (37 levels of
+// TL159: 3.8 MB in and out of each).
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void winds_kernel(const T* __restrict__ x0,
+                                                    const T* __restrict__ x1,
+                                                    T* __restrict__ y0, T* __restrict__ y1,
+                                                    const T* __restrict__ cst,
+                                                    const int* __restrict__ tile_pos,
+                                                    int64_t n_pos, int64_t B, int per, int clip,
+                                                    MP p) {
+  int bx, by;
+  xcd_block(&bx, &by);
+  const int64_t q = (int64_t)bx * blockDim.x + threadIdx.x;
+  if (q >= n_pos) return;
+  const int64_t pos = tile_pos ? tile_pos[q] : q;
+  const int r = (int)(pos / p.L), l = (int)(pos % p.L);
+  const MOff o = moff(p.R, p.L);
+  Stencil<T> S(cst, o, p.R, p.L, r, l);
+  const T inva = (T)(1.0 / p.a);
+  const T il = cst[o.il + l];
+  const T mk = clip ? cst[o.mask + l] : (T)1;
+  const T mk_m = clip ? cst[o.mask + S.lm] : (T)1, mk_p = clip ? cst[o.mask + S.lp] : (T)1;
+  const bool tri = l < ((r + 1) >> 1);  // zero, and what it would read may be unwritten
+  // transposed stencils of the clipped cotangent
+  auto dlon_k = [&](const T* y) -> T { return S.jr * y[S.prow + l] * mk; };
+  auto up_down = [&](const T* y, T up, T dn) -> T {
+    const T a = up * (y[S.row + S.lm] * mk_m), b = dn * (y[S.row + S.lp] * mk_p);
+    return (S.hm ? a : (T)0) + (S.hp ? b : (T)0);
+  };
+  for (int64_t b = (int64_t)by * per; b < B && b < (int64_t)(by + 1) * per; ++b) {
+    const T *u = x0 + b * p.RL, *v = x1 + b * p.RL;
+    T s = 0, t = 0;
+    if (!tri) {
+      if (MODE == 0) {
+        s = (S.dlon(v) * il - S.cldl_il(u)) * inva * mk;
+        t = (S.cldl_il(v) + S.dlon(u) * il) * inva * mk;
+      } else if (MODE == 1) {
+        s = il * ((-up_down(u, S.up_l, S.dn_l) - dlon_k(v)) * inva);
+        t = il * ((-dlon_k(u) + up_down(v, S.up_l, S.dn_l)) * inva);
+      } else if (MODE == 2) {
+        s = (S.dlon(v) - S.sdlc(u)) * inva * mk;
+        t = (S.dlon(u) + S.sdlc(v)) * inva * mk;
+      } else {
+        s = (-up_down(u, S.up2_l, S.dn2_l) - dlon_k(v)) * inva;
+        t = (-dlon_k(u) + up_down(v, S.up2_l, S.dn2_l)) * inva;
+      }
+    }
+    y0[b * p.RL + pos] = s;
+    y1[b * p.RL + pos] = t;
+  }
+}
+
 template <typename T>
 const T* consts(const dino_modal* m) {
   if constexpr (sizeof(T) == 8) return m->c64;
@@ -500,6 +559,31 @@ int run(int which, const dino_modal* m, const void* a, const void* b, void* out,
                                                        epi_groups(m->K, m->nt, moist, E, forced), sg, p);
   }
   DINO_LAUNCH_CHECK("modal kernel");
+  return DINO_OK;
+}
+
+template <typename T>
+int run_winds(int mode, const dino_modal* m, const void* x0, const void* x1, void* y0, void* y1,
+              int64_t B, int clip, hipStream_t s) {
+  const MP p = make_mp(m);
+  int64_t per = 4;  // fields per thread, as the levels of the other modal kernels
+  while ((B + per - 1) / per > 65535) per *= 2;
+  const bool tiles = mode == 0 || mode == 3;  // outputs the inverse transform reads
+  const int64_t n = tiles ? m->n_tile_pos : p.RL;
+  const dim3 grid((unsigned)((n + 255) / 256), (unsigned)((B + per - 1) / per));
+  const int* tp = tiles ? m->tile_pos : nullptr;
+  const T* c = consts<T>(m);
+#define WINDS(MODE)                                                                         \
+  winds_kernel<T, MODE><<<grid, 256, 0, s>>>((const T*)x0, (const T*)x1, (T*)y0, (T*)y1, c, tp, \
+                                             n, B, (int)per, clip, p)
+  switch (mode) {
+    case 0: WINDS(0); break;
+    case 1: WINDS(1); break;
+    case 2: WINDS(2); break;
+    default: WINDS(3);
+  }
+#undef WINDS
+  DINO_LAUNCH_CHECK("winds kernel");
   return DINO_OK;
 }
 
@@ -624,3 +708,18 @@ MODAL_ENTRY(dino_modal_prep, 0)
 MODAL_ENTRY(dino_modal_prep_adjoint, 1)
 MODAL_ENTRY(dino_modal_epilogue, 2)
 MODAL_ENTRY(dino_modal_epilogue_adjoint, 3)
+
+extern "C" int dino_modal_winds(const dino_modal* m, int mode, const void* x0, const void* x1,
+                                void* y0, void* y1, int64_t batch, int clip, int dtype,
+                                void* stream) {
+  DINO_REQUIRE(m, DINO_EINVAL, "dino_modal_winds: NULL handle");
+  DINO_REQUIRE(mode >= 0 && mode <= 3, DINO_EINVAL, "dino_modal_winds: unknown mode %d", mode);
+  DINO_REQUIRE(batch >= 0 && batch < (int64_t)1 << 31, DINO_EINVAL,
+               "dino_modal_winds: batch out of range");
+  if (batch == 0) return DINO_OK;
+  DINO_REQUIRE(x0 && x1 && y0 && y1, DINO_EINVAL, "dino_modal_winds: NULL buffer");
+  if (dtype == DINO_F64)
+    return run_winds<double>(mode, m, x0, x1, y0, y1, batch, clip, as_stream(stream));
+  DINO_REQUIRE(dtype == DINO_F32, DINO_EINVAL, "unknown dtype %d", dtype);
+  return run_winds<float>(mode, m, x0, x1, y0, y1, batch, clip, as_stream(stream));
+}

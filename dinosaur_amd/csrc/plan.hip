@@ -145,14 +145,17 @@ __global__ void twiddle_kernel(int n, double* tw64, float* tw32) {
   tw32[2 * k + 1] = (float)s;
 }
 
-__global__ void quad_weights_kernel(int I, int J, const double* w, double* q64,
-                                    float* q32) {
+__global__ void latitude_weights_kernel(int I, int J, int stride, const double* x,
+                                        const double* w, double* q64, float* q32) {
   int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= J) return;
   const double pi = 3.14159265358979323846;
-  double q = (2.0 * pi / I) * w[j];
-  q64[j] = q;
-  q32[j] = (float)q;
+  const double q = (2.0 * pi / I) * w[j], sec = 1.0 / sqrt(1.0 - x[j] * x[j]);
+  const double rows[3] = {q, sec, q * sec};
+  for (int i = 0; i < 3; ++i) {
+    q64[i * stride + j] = rows[i];
+    q32[i * stride + j] = (float)rows[i];
+  }
 }
 
 bool dft_mixed_available(int N, bool f64);
@@ -247,8 +250,9 @@ extern "C" int dino_plan_create(int M, int L, int I, int J, const double* nodes,
   } while (0)
   PLAN_HIP(hipMalloc(&p->nodes64, sizeof(double) * J));
   PLAN_HIP(hipMalloc(&p->weights64, sizeof(double) * J));
-  PLAN_HIP(hipMalloc(&p->qw64, sizeof(double) * J));
-  PLAN_HIP(hipMalloc(&p->qw32, sizeof(float) * J));
+  p->qw_stride = (J + 3) / 4 * 4;
+  PLAN_HIP(hipMalloc(&p->qw64, sizeof(double) * 3 * p->qw_stride));
+  PLAN_HIP(hipMalloc(&p->qw32, sizeof(float) * 3 * p->qw_stride));
   PLAN_HIP(hipMalloc(&p->m_offset, sizeof(int64_t) * M));
   PLAN_HIP(hipMalloc(&p->p64, sizeof(double) * acc));
   PLAN_HIP(hipMalloc(&p->p32, sizeof(float) * acc));
@@ -264,7 +268,8 @@ extern "C" int dino_plan_create(int M, int L, int I, int J, const double* nodes,
     gauss_nodes_kernel<<<(half + 63) / 64, 64>>>(J, p->nodes64, p->weights64);
     PLAN_HIP(hipGetLastError());
   }
-  quad_weights_kernel<<<(J + 255) / 256, 256>>>(I, J, p->weights64, p->qw64, p->qw32);
+  latitude_weights_kernel<<<(J + 255) / 256, 256>>>(I, J, p->qw_stride, p->nodes64, p->weights64,
+                                                    p->qw64, p->qw32);
   PLAN_HIP(hipGetLastError());
   dim3 tgrid((p->Jhp + 63) / 64, M);
   legendre_table_kernel<<<tgrid, 64>>>(M, L, J, p->Jh, p->Jhp, p->nodes64,

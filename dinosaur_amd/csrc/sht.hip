@@ -59,6 +59,14 @@ bool take_triangle_flag(int* precision) {
   return t;
 }
 
+// Splits the DINO_SHT_SEC_LAT flag off a precision argument: the bit it adds to
+// the longitude kernels' weight code (0 none, 1 quadrature; + 2: / cos(lat)).
+int take_sec_flag(int* precision) {
+  const int w = (*precision & DINO_SHT_SEC_LAT) != 0 ? 2 : 0;
+  *precision &= ~DINO_SHT_SEC_LAT;
+  return w;
+}
+
 // Device address of `scratch` on the current device, looked up once per
 // device (each device has its own copy at its own address).
 constexpr int kScratchDevices = 64;
@@ -92,11 +100,12 @@ int scratch_address(void** out) {
 
 extern "C" int dino_sht_inverse(const dino_plan* p, const void* modal, void* nodal, void* work,
                                 int64_t batch, int dtype, int precision, void* stream) {
+  const int sec = take_sec_flag(&precision);
   CHECK_OR_RETURN(check_common(p, modal, nodal, batch, dtype, precision));
   DINO_REQUIRE(batch == 0 || work, DINO_EINVAL, "NULL workspace");
   hipStream_t s = as_stream(stream);
   CHECK_OR_RETURN(leg_inverse(p, modal, work, batch, dtype, precision, s));
-  return dft_inverse_impl(p, work, nodal, batch, dtype, 0, s);
+  return dft_inverse_impl(p, work, nodal, batch, dtype, sec, s);
 }
 
 // The same kernels as dino_sht_inverse, with the Fourier rows in `scratch`.
@@ -121,10 +130,11 @@ extern "C" int dino_sht_inverse_scratch(const dino_plan* p, const void* modal, v
 extern "C" int dino_sht_forward(const dino_plan* p, const void* nodal, void* modal, void* work,
                                 int64_t batch, int dtype, int precision, void* stream) {
   const bool tri = take_triangle_flag(&precision);
+  const int sec = take_sec_flag(&precision);
   CHECK_OR_RETURN(check_common(p, nodal, modal, batch, dtype, precision));
   DINO_REQUIRE(batch == 0 || work, DINO_EINVAL, "NULL workspace");
   hipStream_t s = as_stream(stream);
-  CHECK_OR_RETURN(dft_forward_impl(p, nodal, work, batch, dtype, 1, s));
+  CHECK_OR_RETURN(dft_forward_impl(p, nodal, work, batch, dtype, 1 | sec, s));
   return leg_forward(p, work, modal, batch, dtype, precision, s, tri);
 }
 
@@ -132,33 +142,35 @@ extern "C" int dino_sht_inverse_adjoint(const dino_plan* p, const void* nodal_co
                                         void* modal_cot, void* work, int64_t batch, int dtype,
                                         int precision, void* stream) {
   const bool tri = take_triangle_flag(&precision);
+  const int sec = take_sec_flag(&precision);
   CHECK_OR_RETURN(check_common(p, nodal_cot, modal_cot, batch, dtype, precision));
   DINO_REQUIRE(batch == 0 || work, DINO_EINVAL, "NULL workspace");
   hipStream_t s = as_stream(stream);
-  CHECK_OR_RETURN(dft_forward_impl(p, nodal_cot, work, batch, dtype, 0, s));
+  CHECK_OR_RETURN(dft_forward_impl(p, nodal_cot, work, batch, dtype, sec, s));
   return leg_forward(p, work, modal_cot, batch, dtype, precision, s, tri);
 }
 
 extern "C" int dino_sht_forward_adjoint(const dino_plan* p, const void* modal_cot,
                                         void* nodal_cot, void* work, int64_t batch, int dtype,
                                         int precision, void* stream) {
+  const int sec = take_sec_flag(&precision);
   CHECK_OR_RETURN(check_common(p, modal_cot, nodal_cot, batch, dtype, precision));
   DINO_REQUIRE(batch == 0 || work, DINO_EINVAL, "NULL workspace");
   hipStream_t s = as_stream(stream);
   CHECK_OR_RETURN(leg_inverse(p, modal_cot, work, batch, dtype, precision, s));
-  return dft_inverse_impl(p, work, nodal_cot, batch, dtype, 1, s);
+  return dft_inverse_impl(p, work, nodal_cot, batch, dtype, 1 | sec, s);
 }
 
 extern "C" int dino_dft_forward(const dino_plan* p, const void* nodal, void* fourier,
                                 int64_t batch, int dtype, int weighted, void* stream) {
   CHECK_OR_RETURN(check_common(p, nodal, fourier, batch, dtype, DINO_PREC_NATIVE));
-  return dft_forward_impl(p, nodal, fourier, batch, dtype, weighted, as_stream(stream));
+  return dft_forward_impl(p, nodal, fourier, batch, dtype, weighted ? 1 : 0, as_stream(stream));
 }
 
 extern "C" int dino_dft_inverse(const dino_plan* p, const void* fourier, void* nodal,
                                 int64_t batch, int dtype, int weighted, void* stream) {
   CHECK_OR_RETURN(check_common(p, fourier, nodal, batch, dtype, DINO_PREC_NATIVE));
-  return dft_inverse_impl(p, fourier, nodal, batch, dtype, weighted, as_stream(stream));
+  return dft_inverse_impl(p, fourier, nodal, batch, dtype, weighted ? 1 : 0, as_stream(stream));
 }
 
 extern "C" int dino_legendre_inverse(const dino_plan* p, const void* modal, void* fourier,

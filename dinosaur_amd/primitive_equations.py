@@ -568,6 +568,26 @@ class _Handle:
       pass
 
 
+def modal_handle(grid, layers, tracers, humidity, gravity, device, flags=0) -> _Handle:
+  """dino_modal of a grid: the coefficients of its derivative and Laplacian
+  operators on a device (spherical_harmonic.py:1033-1092)."""
+  R, L = grid.modal_shape
+  f64 = lambda a: np.ascontiguousarray(np.asarray(a, np.float64))
+  mask = np.ones(L)
+  mask[-1] = 0.0
+  arrays = [f64(spherical_harmonic._grid_host_const(grid, 'inverse_laplacian')),
+            f64(grid.laplacian_eigenvalues), f64(mask)]
+  arrays += [f64(spherical_harmonic._grid_host_const(grid, n))
+             for n in ('cdlat_up', 'cdlat_dn', 'scdlat_up', 'scdlat_dn')]
+  handle = ctypes.c_void_p()
+  with torch.cuda.device(device):
+    rc = _lib.lib().dino_modal_create_ex(
+        R, L, layers, tracers, humidity, float(grid.radius), float(gravity),
+        *(_lib.dptr(a) for a in arrays), flags, ctypes.byref(handle))
+  _lib.check(rc, 'dino_modal_create_ex')
+  return _Handle(handle, 'dino_modal_destroy')
+
+
 def _launch(name, h, a, b, out, members, like):
   code = _lib.DINO_F64 if like.dtype == torch.float64 else _lib.DINO_F32
   stream = ctypes.c_void_p(torch.cuda.current_stream(like.device).cuda_stream)
@@ -880,28 +900,11 @@ class PrimitiveEquationsSigma:
     key = (torch.device(device).index, tuple(names), flags)
     cache = self.__dict__.setdefault('_modal_handles', {})
     h = cache.get(key)
-    if h is not None:
-      return h
-    grid = self.coords.horizontal
-    R_, L_ = grid.modal_shape
-    f64 = lambda a: np.ascontiguousarray(np.asarray(a, np.float64))
-    il = f64(spherical_harmonic._grid_host_const(grid, 'inverse_laplacian'))
-    ev = f64(grid.laplacian_eigenvalues)
-    mask = np.ones(L_)
-    mask[-1] = 0.0
-    cst = [f64(spherical_harmonic._grid_host_const(grid, n))
-           for n in ('cdlat_up', 'cdlat_dn', 'scdlat_up', 'scdlat_dn')]
-    hum = names.index(self.humidity_key) if self.humidity_key is not None else -1
-    handle = ctypes.c_void_p()
-    dp = _lib.dptr
-    with torch.cuda.device(device):
-      rc = _lib.lib().dino_modal_create_ex(
-          R_, L_, self.coords.vertical.layers, len(names), hum, float(grid.radius),
-          float(self.physics_specs.g), dp(il), dp(ev), dp(f64(mask)), *(dp(c) for c in cst),
-          flags, ctypes.byref(handle))
-    _lib.check(rc, 'dino_modal_create_ex')
-    h = _Handle(handle, 'dino_modal_destroy')
-    cache[key] = h
+    if h is None:
+      hum = names.index(self.humidity_key) if self.humidity_key is not None else -1
+      h = modal_handle(self.coords.horizontal, self.coords.vertical.layers, len(names), hum,
+                       float(self.physics_specs.g), device, flags)
+      cache[key] = h
     return h
 
   def _check_tracers(self, state):
@@ -1454,33 +1457,8 @@ class PrimitiveEquationsHybrid(PrimitiveEquationsSigma):
     cache[key] = h
     return h
 
-  def _modal_handle(self, device, names):
-    key = (torch.device(device).index, tuple(names))
-    cache = self.__dict__.setdefault('_modal_handles', {})
-    h = cache.get(key)
-    if h is not None:
-      return h
-    grid = self.coords.horizontal
-    R_, L_ = grid.modal_shape
-    f64 = lambda a: np.ascontiguousarray(np.asarray(a, np.float64))
-    il = f64(spherical_harmonic._grid_host_const(grid, 'inverse_laplacian'))
-    ev = f64(grid.laplacian_eigenvalues)
-    mask = np.ones(L_)
-    mask[-1] = 0.0
-    cst = [f64(spherical_harmonic._grid_host_const(grid, n))
-           for n in ('cdlat_up', 'cdlat_dn', 'scdlat_up', 'scdlat_dn')]
-    hum = names.index(self.humidity_key) if self.humidity_key is not None else -1
-    handle = ctypes.c_void_p()
-    dp = _lib.dptr
-    with torch.cuda.device(device):
-      rc = _lib.lib().dino_modal_create_ex(
-          R_, L_, self.coords.vertical.layers, len(names), hum, float(grid.radius),
-          float(self.physics_specs.g), dp(il), dp(ev), dp(f64(mask)), *(dp(c) for c in cst),
-          _lib.MODAL_HYBRID, ctypes.byref(handle))
-    _lib.check(rc, 'dino_modal_create_ex')
-    h = _Handle(handle, 'dino_modal_destroy')
-    cache[key] = h
-    return h
+  def _modal_handle(self, device, names, flags=0):
+    return super()._modal_handle(device, names, flags | _lib.MODAL_HYBRID)
 
   def _explicit_fused(self, state: State, names) -> State:
     """As the sigma path, with the hybrid nodal kernel between the transforms."""

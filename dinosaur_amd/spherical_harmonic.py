@@ -204,8 +204,8 @@ def sht_call(fn_name: str, plan: Plan, x: torch.Tensor, out_tail: tuple, precisi
   if batch == 0:
     return out
   work = _workspace(plan, batch, x)
-  flags = precision & _lib.SHT_TRIANGLE_ONLY
-  precision &= ~_lib.SHT_TRIANGLE_ONLY
+  flags = precision & (_lib.SHT_TRIANGLE_ONLY | _lib.SHT_SEC_LAT)
+  precision &= ~flags
   if x.dtype == torch.float64:
     precision = _lib.PREC_NATIVE  # FP64 data always runs FP64 arithmetic
   plan.apply_tuned(batch, _dtype_code(x), precision)
@@ -1002,10 +1002,78 @@ def get_cos_lat_vector(vorticity, divergence, grid: Grid, clip: bool = True):
   return (a[0] + b[0], a[1] + b[1])
 
 
+class _Winds(torch.autograd.Function):
+  """One direction of dino_modal_winds on two (B, 2M-1, L) tensors a and b, or
+  on the halves of a (2B, 2M-1, L) tensor a (b None) -> (2B, 2M-1, L); the
+  backward is its adjoint mode."""
+
+  @staticmethod
+  def _run(handle, mode, a, b, clip):
+    a = a.contiguous()
+    B, tail = a.shape[0] // (2 if b is None else 1), tuple(a.shape[1:])
+    b = a[B:] if b is None else b.contiguous()
+    out = torch.empty((2 * B,) + tail, dtype=a.dtype, device=a.device)
+    with torch.cuda.device(a.device):
+      rc = _lib.lib().dino_modal_winds(handle.handle, mode, _ptr(a), _ptr(b), _ptr(out),
+                                       _ptr(out[B:]), B, int(clip), _dtype_code(a),
+                                       _stream(a.device))
+    _lib.check(rc, 'dino_modal_winds')
+    if _lib._active is not None:
+      _lib.tally('winds', a.element_size() * 4 * B * _lib.triangle_entries(*tail))
+    return out
+
+  @staticmethod
+  def forward(ctx, a, b, handle, mode, clip):
+    ctx.handle, ctx.mode, ctx.clip, ctx.pair = handle, mode, clip, b is None
+    return _Winds._run(handle, mode, a, b, clip)
+
+  @staticmethod
+  def backward(ctx, g):
+    gin = _Winds._run(ctx.handle, ctx.mode + 1, g, None, ctx.clip)
+    if ctx.pair:
+      return gin, None, None, None, None
+    B = gin.shape[0] // 2
+    return gin[:B], gin[B:], None, None, None
+
+
+def _pair_of(x, lead, tail):
+  """The two fields of a (2B, ...) buffer; tensors of their own when autograd
+  follows them, so that one may be changed in place without the other."""
+  a, b = (x[i * (x.shape[0] // 2):(i + 1) * (x.shape[0] // 2)].reshape(lead + tail)
+          for i in (0, 1))
+  return (a.clone(), b.clone()) if x.requires_grad else (a, b)
+
+
+def _winds_handle(grid: Grid, a: torch.Tensor, b: torch.Tensor, tail):
+  """The grid's operator handle when the fused wind kernels serve this pair of
+  tensors (Real layout, one shape, float type and device), else None."""
+  sh = grid.spherical_harmonics
+  if (type(sh) is not RealSphericalHarmonics or a.shape != b.shape or a.dtype != b.dtype
+      or a.device != b.device or a.dtype not in (torch.float32, torch.float64)
+      or tuple(a.shape[-2:]) != tuple(tail) or a.numel() == 0):
+    return None
+  key = (grid, 'winds', a.device)
+  h = _const_cache.get(key)
+  if h is None:
+    from .primitive_equations import modal_handle  # pylint: disable=import-outside-toplevel
+    h = modal_handle(grid, 1, 0, -1, 0.0, a.device)
+    _const_cache[key] = h
+  return h
+
+
 def uv_nodal_to_vor_div_modal(grid: Grid, u_nodal, v_nodal, clip: bool = True):
   """spherical_harmonic.py:1181-1195."""
   u, restore = _as_tensor(u_nodal)
   v, _ = _as_tensor(v_nodal)
+  handle = _winds_handle(grid, u, v, grid.nodal_shape)
+  if handle is not None:
+    # the division by cos(lat) is in the transform's quadrature weights
+    sh, lead = grid.spherical_harmonics, u.shape[:-2]
+    pair = torch.stack([u, v]).reshape((-1,) + grid.nodal_shape)
+    modal = _ToModal.apply(pair, sh.plan(u.device), sh._precision | _lib.SHT_SEC_LAT, True)
+    vd = _Winds.apply(modal, None, handle, _lib.WINDS_TO_VOR_DIV, clip)
+    vort, div = _pair_of(vd, lead, grid.modal_shape)
+    return restore(vort), restore(div)
   cos = grid.const('cos_lat', u.device, u.dtype)
   uc, vc = grid.to_modal_batched([u / cos, v / cos])
   return (restore(grid.curl_cos_lat((uc, vc), clip=clip)),
@@ -1016,6 +1084,15 @@ def vor_div_to_uv_nodal(grid: Grid, vorticity, divergence, clip: bool = True):
   """spherical_harmonic.py:1198-1210."""
   z, restore = _as_tensor(vorticity)
   d, _ = _as_tensor(divergence)
+  handle = _winds_handle(grid, z, d, grid.modal_shape)
+  if handle is not None:
+    # the division by cos(lat) is in the transform's last pass
+    sh, lead = grid.spherical_harmonics, z.shape[:-2]
+    flat = (-1,) + grid.modal_shape
+    modal = _Winds.apply(z.reshape(flat), d.reshape(flat), handle, _lib.WINDS_FROM_VOR_DIV, clip)
+    uv = _ToNodal.apply(modal, sh.plan(z.device), sh._precision | _lib.SHT_SEC_LAT, True)
+    un, vn = _pair_of(uv, lead, grid.nodal_shape)
+    return restore(un), restore(vn)
   u, v = get_cos_lat_vector(z, d, grid, clip=clip)
   un, vn = grid.to_nodal_batched([u, v])
   cos = grid.const('cos_lat', un.device, un.dtype)

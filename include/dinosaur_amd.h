@@ -44,6 +44,11 @@ enum {
   DINO_PREC_BF16X3 = 2, /* split-BF16 x3 on MFMA, FP32 accumulation */
 };
 
+/* Flag or-ed into `precision` of dino_sht_inverse, dino_sht_forward and their
+ * adjoints: nodal values are divided by cos(lat), after the inverse and before
+ * the forward transform, in the longitude kernels' weights. */
+enum { DINO_SHT_SEC_LAT = 0x200 };
+
 /* Flag or-ed into `precision` of dino_sht_forward, dino_sht_inverse_adjoint
  * and dino_legendre_forward: each modal row of zonal wavenumber m is written
  * only from degree s(m) = max(0, L - 32 * ceil((L - m) / 32)) on (the first
@@ -467,6 +472,24 @@ int dino_modal_create_ex(int R, int L, int K, int n_tracers, int humidity_index,
                          const double* lap, const double* clip_mask,
                          const double* up, const double* dn, const double* up2,
                          const double* dn2, int flags, dino_modal** out);
+
+/* Vorticity and divergence <-> winds times cos(lat) in the modal basis
+ * (dinosaur/spherical_harmonic.py:1164-1210), (batch, 2M-1, L) buffers:
+ *   DINO_WINDS_FROM_VOR_DIV: x0 = vorticity, x1 = divergence -> y0 = u cos(lat),
+ *     y1 = v cos(lat);   ..._ADJOINT: x = cotangents of those -> y of the inputs
+ *   DINO_WINDS_TO_VOR_DIV: x0, x1 = transforms of u / cos(lat), v / cos(lat) ->
+ *     y0 = vorticity, y1 = divergence;   ..._ADJOINT likewise.
+ * clip: zero the top degree of the forward modes' outputs.  FROM_VOR_DIV and
+ * TO_VOR_DIV_ADJOINT write only the degrees that dino_sht_inverse reads. */
+enum {
+  DINO_WINDS_FROM_VOR_DIV = 0,
+  DINO_WINDS_FROM_VOR_DIV_ADJOINT = 1,
+  DINO_WINDS_TO_VOR_DIV = 2,
+  DINO_WINDS_TO_VOR_DIV_ADJOINT = 3,
+};
+int dino_modal_winds(const dino_modal* m, int mode, const void* x0,
+                     const void* x1, void* y0, void* y1, int64_t batch,
+                     int clip, int dtype, void* stream);
 
 /* Fused nodal nonlinear terms of PrimitiveEquationsHybrid.explicit_terms.
  * Replaces compute_diagnostic_state_hybrid, the Simmons-Burridge
