@@ -16,6 +16,10 @@ int dft_forward_impl(const dino_plan*, const void*, void*, int64_t, int, int, hi
 int dft_inverse_impl(const dino_plan*, const void*, void*, int64_t, int, int, hipStream_t);
 int legendre_inverse_fma(const dino_plan*, const void*, void*, int64_t, int, hipStream_t);
 int legendre_forward_fma(const dino_plan*, const void*, void*, int64_t, int, hipStream_t);
+bool legendre_f64_forward_pays(const dino_plan*, int64_t);
+bool legendre_f64_inverse_pays(const dino_plan*, int64_t);
+int legendre_inverse_f64(const dino_plan*, const double*, double*, int64_t, hipStream_t);
+int legendre_forward_f64(const dino_plan*, const double*, double*, int64_t, bool, hipStream_t);
 int legendre_inverse_mfma(const dino_plan*, const void*, void*, int64_t, int, hipStream_t);
 int legendre_forward_mfma(const dino_plan*, const void*, void*, int64_t, int, bool, hipStream_t);
 }  // namespace dino
@@ -37,9 +41,12 @@ int check_common(const dino_plan* p, const void* a, const void* b, int64_t batch
   return DINO_OK;
 }
 
-// FP64 data: FP64 FMA tiles.  FP32 data: MFMA (FP32 or split BF16 x3).
+// FP64 data: FP64 MFMA, or FMA tiles where they are faster (legendre_f64.hip).
+// FP32 data: MFMA (FP32 or split BF16 x3).
 int leg_inverse(const dino_plan* p, const void* in, void* out, int64_t B, int dtype, int prec,
                 hipStream_t s) {
+  if (dtype == DINO_F64 && legendre_f64_inverse_pays(p, B))
+    return legendre_inverse_f64(p, static_cast<const double*>(in), static_cast<double*>(out), B, s);
   if (dtype == DINO_F64) return legendre_inverse_fma(p, in, out, B, dtype, s);
   return legendre_inverse_mfma(p, in, out, B, prec, s);
 }
@@ -48,6 +55,9 @@ int leg_inverse(const dino_plan* p, const void* in, void* out, int64_t B, int dt
 // (the FP64 and tiled kernels write them anyway, which is also allowed).
 int leg_forward(const dino_plan* p, const void* in, void* out, int64_t B, int dtype, int prec,
                 hipStream_t s, bool triangle_only = false) {
+  if (dtype == DINO_F64 && legendre_f64_forward_pays(p, B))
+    return legendre_forward_f64(p, static_cast<const double*>(in), static_cast<double*>(out), B,
+                                triangle_only, s);
   if (dtype == DINO_F64) return legendre_forward_fma(p, in, out, B, dtype, s);
   return legendre_forward_mfma(p, in, out, B, prec, triangle_only, s);
 }
