@@ -38,6 +38,25 @@ _c_i64 = ctypes.c_int64
 _c_d = ctypes.c_double
 _c_dp = ctypes.POINTER(ctypes.c_double)
 
+
+
+class ExplicitArgs(ctypes.Structure):
+  """dino_explicit_args."""
+  _fields_ = [('plan', _c_p), ('modal', _c_p), ('nodal', _c_p), ('forcing', _c_p),
+              ('orography', _c_p), ('members', _c_i64), ('layers', _c_i), ('tracers', _c_i),
+              ('dtype', _c_i), ('precision', _c_i)]
+
+
+class ImexStepArgs(ctypes.Structure):
+  """dino_imex_step_args."""
+  _fields_ = [('explicit_args', ExplicitArgs), ('stages', _c_i), ('degrees', _c_i),
+              ('triangle_only', _c_i), ('reserved', _c_i), ('a_ex', _c_dp), ('a_im', _c_dp),
+              ('b_ex', _c_dp), ('b_im', _c_dp), ('dt', _c_d), ('terms', _c_p),
+              ('solve', ctypes.POINTER(_c_p)), ('n', _c_i64), ('im_begin', _c_i64),
+              ('im_end', _c_i64), ('g_origin', _c_i64), ('field_size', _c_i64),
+              ('scale_len', _c_i64), ('degree_scale', _c_p)]
+
+
 # name -> (restype, argtypes); every symbol declared in include/dinosaur_amd.h
 SIGNATURES = {
     'dino_last_error': (ctypes.c_char_p, []),
@@ -114,6 +133,10 @@ SIGNATURES = {
     'dino_held_suarez_nodal': (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i, _c_p]),
     'dino_held_suarez_nodal_adjoint': (_c_i, [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i,
                                               _c_p]),
+    'dino_explicit_workspace': (_c_i64, [ctypes.POINTER(ExplicitArgs)]),
+    'dino_explicit_terms': (_c_i, [ctypes.POINTER(ExplicitArgs), _c_p, _c_p, _c_p, _c_p]),
+    'dino_imex_step_workspace': (_c_i64, [ctypes.POINTER(ImexStepArgs)]),
+    'dino_imex_step': (_c_i, [ctypes.POINTER(ImexStepArgs), _c_p, _c_p, _c_p, _c_p]),
     'dino_vregrid_create': (_c_i, [_c_i, _c_i, _c_dp, _c_dp, _c_i, _c_dp, _c_dp,
                                    ctypes.POINTER(_c_p)]),
     'dino_vregrid_destroy': (_c_i, [_c_p]),

@@ -153,5 +153,9 @@ class _ForcedEquations:
   def flat_imex_ops(self, state):
     ops = self.equation._flat_imex_ops(state)
     if ops is not None:
+      eq, members, names = self.equation, ops.members, ops.names
       ops.explicit_terms = self.explicit_terms
+      if ops.native_args is not None:
+        ops.native_args = lambda buf: eq._native_args(buf, members, eq._check_names(names),
+                                                      self.forcing)
     return ops

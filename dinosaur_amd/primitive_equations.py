@@ -681,6 +681,23 @@ class _ImplicitFlat(torch.autograd.Function):
     return gin, None, None, None, None, None
 
 
+# Largest workspace of the one-call paths.  Beyond it a launch runs long enough
+# (T85 L24, 2 members: 60-130 us each) that the host keeps ahead of the GPU, and
+# the separate calls hold less memory at a time.
+_NATIVE_WORK_BYTES = 256 << 20
+
+
+def _plain(buf: torch.Tensor) -> bool:
+  """Whether a result may be formed outside autograd: no gradient is recorded,
+  and no forward-mode or functorch transform is active (the autograd functions
+  of the separate calls raise under those)."""
+  return (type(buf) is torch.Tensor and not (torch.is_grad_enabled() and buf.requires_grad)
+          and torch.autograd.forward_ad._current_level < 0
+          and torch._C._functorch.maybe_current_level() is None
+          and not torch.jit.is_tracing()
+          and _lib._active is None and not _lib.skip_values())
+
+
 class _FlatImexOps:
   """Flat-buffer operations of one state layout for the fused IMEX step
   (time_integration._fused_imex_step): explicit terms (differentiable),
@@ -709,6 +726,12 @@ class _FlatImexOps:
     self.n = (3 * E * K + E + E * K * len(names)) * self.RL
     self.op = eq._implicit
     self.explicit_terms = eq.explicit_terms
+    # arguments of the one-call explicit terms on a flat buffer, if they are
+    # the equation's own
+    fused = (eq.fused_nodal and 'explicit_terms' not in eq.__dict__ and
+             type(eq).explicit_terms is PrimitiveEquationsSigma.explicit_terms)
+    self.native_args = ((lambda buf: eq._native_args(buf, members, eq._check_names(names)))
+                        if fused else None)
     # Real layout: the stage kernels skip the all-zero part l < m of each field
     real = isinstance(eq.coords.horizontal.spherical_harmonics,
                       spherical_harmonic.RealSphericalHarmonics)
@@ -721,6 +744,38 @@ class _FlatImexOps:
     # multiply those entries by zero coefficients.
     self.stage_triangle_only = (real and eq.fused_nodal and
                                 type(eq).explicit_terms is PrimitiveEquationsSigma.explicit_terms)
+
+  def native_step(self, buf, tab, dt, scale):
+    """One whole step in one call (dino_imex_step), or None where that does not
+    apply (see _native_args, _NATIVE_WORK_BYTES)."""
+    ex = self.native_args(buf) if self.native_args is not None else None
+    if ex is None or not _plain(buf):
+      return None
+    n = len(tab.b_ex)
+    table = lambda rows: (ctypes.c_double * len(rows))(*rows)  # noqa: E731
+    a_ex = table([c for i in range(n - 1)
+                  for c in list(tab.a_ex[i]) + [0.0] * (n - len(tab.a_ex[i]))])
+    a_im = table([c for i in range(n - 1)
+                  for c in list(tab.a_im[i]) + [0.0] * (n - len(tab.a_im[i]))])
+    b_ex, b_im = table(list(tab.b_ex)), table(list(tab.b_im))
+    solve = (ctypes.c_void_p * (n - 1))(
+        *[self.op.factor(float(dt * tab.a_im[i][i + 1]), buf.device) for i in range(n - 1)])
+    args = _lib.ImexStepArgs(
+        ex, n, self.degrees, int(self.stage_triangle_only), 0, a_ex, a_im, b_ex, b_im, float(dt),
+        self.op.factor(0.0, buf.device), solve, self.n, self.ib, self.ie, self.go,
+        self.field_size, scale.numel() if scale is not None else 0,
+        scale.data_ptr() if scale is not None else None)
+    lib = _lib.lib()
+    size = lib.dino_imex_step_workspace(ctypes.byref(args))
+    if not 0 < size * buf.element_size() <= _NATIVE_WORK_BYTES:
+      return None
+    out = torch.empty_like(buf)
+    work = torch.empty(size, dtype=buf.dtype, device=buf.device)
+    with torch.cuda.device(buf.device):
+      rc = lib.dino_imex_step(ctypes.byref(args), buf.data_ptr(), out.data_ptr(), work.data_ptr(),
+                              torch.cuda.current_stream(buf.device).cuda_stream)
+    _lib.check(rc, 'dino_imex_step')
+    return out
 
   def state(self, buf):
     return State.from_flat(buf, *self.layout)
@@ -908,11 +963,12 @@ class PrimitiveEquationsSigma:
     return h
 
   def _check_tracers(self, state):
-    names = list(state.tracers.keys())
-    if self.humidity_key is not None and self.humidity_key not in state.tracers:
-      raise ValueError(f'`{self.humidity_key}` is not found in tracers: {names}.')
-    for key in self.cloud_keys or ():
-      if key not in state.tracers:
+    return self._check_names(state.tracers.keys())
+
+  def _check_names(self, names):
+    names = list(names)
+    for key in (self.humidity_key, *(self.cloud_keys or ())):
+      if key is not None and key not in names:
         raise ValueError(f'`{key}` is not found in tracers: {names}.')
     return names
 
@@ -1047,6 +1103,20 @@ class PrimitiveEquationsSigma:
     buf = flat.flat_buffer()
     lead, K, _ = flat._flat[1:]
     members = int(np.prod(lead)) if lead else 1
+    args = self._native_args(buf, members, names, forcing)
+    if args is not None:
+      lib = _lib.lib()
+      n = lib.dino_explicit_workspace(ctypes.byref(args))
+      if 0 < n * buf.element_size() <= _NATIVE_WORK_BYTES:
+        tend = torch.empty_like(buf)
+        work = torch.empty(n, dtype=buf.dtype, device=buf.device)
+        with torch.cuda.device(buf.device):
+          rc = lib.dino_explicit_terms(
+              ctypes.byref(args), buf.data_ptr(), tend.data_ptr(), work.data_ptr(),
+              torch.cuda.current_stream(buf.device).cuda_stream)
+        _lib.check(rc, 'dino_explicit_terms')
+        return State.from_flat(tend, lead, K, names,
+                               sim_time=None if state.sim_time is None else 1.0)
     mh = self._modal_handle(buf.device, names, _lib.MODAL_FORCED if forcing is not None else 0)
     prep = _ModalPrep.apply(buf, mh, members)
     # the modal buffers between the transforms and the prep / epilogue kernels
@@ -1065,6 +1135,31 @@ class PrimitiveEquationsSigma:
     tend = _ModalEpilogue.apply(mod, mh, members, self._orography_modal(buf).contiguous())
     return State.from_flat(tend, lead, K, names,
                            sim_time=None if state.sim_time is None else 1.0)
+
+  def _native_args(self, buf, members, names, forcing=None):
+    """Arguments of the one-call explicit terms on a flat state buffer, or None
+    where they do not apply: under autograd and its transforms, with tuned
+    launch schedules (set per transform and batch), or replaced methods or
+    transforms.  The tensors and handles they point to live in this object's
+    caches and the caller's buffers."""
+    sh = self.coords.horizontal.spherical_harmonics
+    if (type(sh) is not spherical_harmonic.RealSphericalHarmonics or not _plain(buf)
+        or type(self)._explicit_fused is not PrimitiveEquationsSigma._explicit_fused
+        or not buf.is_contiguous() or buf.dtype not in (torch.float32, torch.float64)):
+      return None
+    plan = sh.plan(buf.device)
+    if plan.tuned:
+      return None
+    flags = _lib.MODAL_FORCED if forcing is not None else 0
+    oro = self._orography_modal(buf)
+    if not oro.is_contiguous():
+      return None
+    return _lib.ExplicitArgs(
+        plan.handle, self._modal_handle(buf.device, names, flags).handle,
+        self._nodal_handle(buf.device, names).handle,
+        forcing.handle(buf.device).handle if forcing is not None else None, oro.data_ptr(),
+        members, self.coords.vertical.layers, len(names),
+        _lib.DINO_F64 if buf.dtype == torch.float64 else _lib.DINO_F32, sh._precision)
 
   @property
   def _modal_moist(self) -> bool:

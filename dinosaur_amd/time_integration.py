@@ -518,7 +518,10 @@ def _fused_imex_step(ops, tab, dt, y0, out_scale=None):
     out = _FusedImexStep.apply(ops, tab, dt, buf, out_scale, need)
   else:
     with torch.no_grad():
-      out = _fused_forward(ops, tab, dt, buf, keep=False, out_scale=out_scale)[0]
+      native = getattr(ops, 'native_step', None)
+      out = native(buf, tab, dt, out_scale) if native is not None else None
+      if out is None:
+        out = _fused_forward(ops, tab, dt, buf, keep=False, out_scale=out_scale)[0]
   t0 = y0.sim_time
   st = None
   if t0 is not None:

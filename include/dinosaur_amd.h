@@ -551,6 +551,47 @@ int dino_held_suarez_nodal_adjoint(const dino_held_suarez* h,
                                    const int64_t* out_groups, int64_t members,
                                    int dtype, void* stream);
 
+/* One evaluation of the sigma equations' explicit terms
+ * (primitive_equations.py:1126-1194): dino_modal_prep, dino_sht_inverse,
+ * dino_nodal_explicit, the forcing if any (modal made with DINO_MODAL_FORCED),
+ * dino_sht_forward and dino_modal_epilogue, on a workspace of
+ * dino_explicit_workspace elements of the data type (-1: invalid arguments). */
+typedef struct dino_explicit_args {
+  const dino_plan* plan;
+  const dino_modal* modal;
+  const dino_nodal* nodal;
+  const dino_held_suarez* forcing; /* or NULL */
+  const void* orography;           /* (2M-1, L) */
+  int64_t members;
+  int layers, tracers, dtype, precision;
+} dino_explicit_args;
+int64_t dino_explicit_workspace(const dino_explicit_args* args);
+int dino_explicit_terms(const dino_explicit_args* args, const void* state,
+                        void* tendency, void* work, void* stream);
+
+/* One IMEX Runge-Kutta step on a flat state (time_integration.py:313-405) of n
+ * elements, with implicit terms on the range [im_begin, im_end) kept in compact
+ * buffers from g_origin on, as dino_imex_stage_ranged takes them.  a_ex, a_im:
+ * (stages - 1, stages) row-major, b_ex, b_im: stages; at most 4 nonzero terms
+ * per row and kind.  terms: the factor of the implicit terms; solve[i - 1]:
+ * that of stage i, for eta = dt a_im[i - 1][i].  triangle_only: stage values
+ * may leave the entries below the triangle unwritten.  degree_scale: a step
+ * filter's per-degree factors (scale_len), or NULL.  The workspace holds
+ * dino_imex_step_workspace elements; out must not overlap y0. */
+typedef struct dino_imex_step_args {
+  dino_explicit_args explicit_args;
+  int stages, degrees, triangle_only, reserved;
+  const double *a_ex, *a_im, *b_ex, *b_im;
+  double dt;
+  const dino_implicit* terms;
+  const dino_implicit* const* solve;
+  int64_t n, im_begin, im_end, g_origin, field_size, scale_len;
+  const void* degree_scale;
+} dino_imex_step_args;
+int64_t dino_imex_step_workspace(const dino_imex_step_args* args);
+int dino_imex_step(const dino_imex_step_args* args, const void* y0, void* out,
+                   void* work, void* stream);
+
 /* Vertical regridding of nodal columns from hybrid levels (source: K_s
  * layers with interface coefficients a, b, p = a + b ps) to target levels.
  * Modes:
