@@ -72,6 +72,12 @@ __host__ __device__ inline COff coff(int K, int J) {
 
 constexpr int MAXTR = 6;
 
+// Waves that share a column's levels in the split forward kernel, two levels each at
+// least, and the batches it takes (measured at the kernel).
+constexpr int kNodalWaves = 8;
+inline int nodal_waves(int K) { return K / 2 < 1 ? 1 : K / 2 < kNodalWaves ? K / 2 : kNodalWaves; }
+inline bool nodal_split(int64_t columns) { return columns <= 98304; }
+
 struct Groups {
   // input group offsets (in fields of I*J) for member stride computation
   int64_t z, d, t, tr[MAXTR], u, v, gx, gy, lp, qx, qy;
@@ -133,22 +139,39 @@ struct Params {
 };
 
 // ---------------------------------------------------------------- forward
-template <typename T>
-__global__ __launch_bounds__(256) void nodal_forward_kernel(
+// Pass A forms the column totals, pass B streams the levels with a (k, k + 1)
+// window.  A thread walks all levels of its column, or (SPLIT) a block owns 64
+// columns and each of its waves a contiguous share of the levels: a wave's
+// sums meet the others' in LDS, its prefix sums start from those of the waves
+// above and the flux through its top interface is formed from the level above.
+// Whole columns stream every field once, in order, at the copy rate, but a grid
+// of a few thousand columns is then a few dozen waves in a long chain: T42
+// L24, one member (8192 columns), 31 us whole and 16 split; T85 L24 moist, 2
+// members (65536), 73 and 46; TL255 L37 moist, one member (131072), 170 and 192.
+template <typename T, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_kernel(
     const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ cst, Groups g,
     Params p) {
-  const int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int lane = threadIdx.x, wave = SPLIT ? (int)threadIdx.y : 0;
+  const int G = SPLIT ? (int)blockDim.y : 1;
+  const int64_t col = (int64_t)blockIdx.x * blockDim.x + lane;
   const int64_t e = blockIdx.y;
-  if (col >= p.IJ) return;
-  const int K = p.K;
-  const COff o = coff(K, p.J);
-  const int j = (int)(col % p.J);
   const int64_t IJ = p.IJ;
+  // SPLIT: lanes past the last column work on it (barriers) and store nothing
+  if (!SPLIT && col >= IJ) return;
+  const bool ok = !SPLIT || col < IJ;
+  const int64_t cc = ok ? col : IJ - 1;
+  const int K = p.K;
+  const int k0 = SPLIT ? K * wave / G : 0, k1 = SPLIT ? K * (wave + 1) / G : K;  // its levels
+  const COff o = coff(K, p.J);
+  const int j = (int)(cc % p.J);
   // field (group offset, levels) of member e at level k
   auto I_ = [&](int64_t off, int lev, int k) -> const T* {
-    return in + (off + e * lev + k) * IJ + col;
+    return in + (off + e * lev + k) * IJ + cc;
   };
-  auto O_ = [&](int64_t off, int lev, int k) -> T* { return out + (off + e * lev + k) * IJ + col; };
+  auto put = [&](int64_t off, int lev, int k, T v) {
+    if (ok) out[(off + e * lev + k) * IJ + cc] = v;
+  };
   const T s = cst[o.sec2 + j];
   const T fc = cst[o.cor + j];
   const T gx = *I_(g.gx, 1, 0);
@@ -156,9 +179,9 @@ __global__ __launch_bounds__(256) void nodal_forward_kernel(
   const T R = (T)p.R, kappa = (T)p.kappa;
   const bool moist = p.moist != 0;
   const T lp = moist ? *I_(g.lp, 1, 0) : (T)0;
-  // ---- pass A: column totals
+  // ---- pass A: sums of this thread's levels
   T TE = 0, TF = 0, GT = 0;
-  for (int k = 0; k < K; ++k) {
+  auto sum_level = [&](int k) {
     T u = *I_(g.u, K, k), v = *I_(g.v, K, k), d = *I_(g.d, K, k);
     T A = (u * gx + v * gy) * s;
     T ds = cst[o.dsig + k];
@@ -169,21 +192,58 @@ __global__ __launch_bounds__(256) void nodal_forward_kernel(
       T td = q * (t + cst[o.tref + k]) * (T)p.gcr1;
       GT += cst[o.gp + k] * td;
     }
+  };
+  if constexpr (SPLIT) {
+#pragma unroll 4
+    for (int k = k0; k < k1; ++k) sum_level(k);
+  } else {
+    for (int k = 0; k < K; ++k) sum_level(k);
   }
-  *O_(g.lsp, 1, 0) = -TE;
-  // ---- pass B: stream levels with windows (k-1, k, k+1)
-  T PE = 0, PF = 0, PEm = 0, PFm = 0;  // prefixes at k and k-1
-  T Wm = 0, Xm = 0;                     // sigma-dot at interface k-1/2
+  T PE = 0, PF = 0, GP = 0;  // prefixes at k; GP: sum_{1 <= h <= k} gp[h] td[h]
+  if constexpr (SPLIT) {
+    __shared__ T part[3][kNodalWaves][64];
+    part[0][wave][lane] = TE;
+    part[1][wave][lane] = TF;
+    part[2][wave][lane] = GT;
+    __syncthreads();
+    TE = TF = GT = 0;
+    for (int i = 0; i < G; ++i) {
+      if (i == wave) {
+        PE = TE;
+        PF = TF;
+        GP = GT;
+      }
+      TE += part[0][i][lane];
+      TF += part[1][i][lane];
+      GT += part[2][i][lane];
+    }
+  }
+  if (wave == 0) put(g.lsp, 1, 0, -TE);
+  // ---- pass B: stream levels with a window (k, k + 1)
+  T PEm = PE, PFm = PF;  // prefixes at k - 1
   // flux of the previous interface for each advected field: U, V, T, tracers
   T fu_m = 0, fv_m = 0, ft_m = 0, fx_m = 0, ftr_m[MAXTR];
 #pragma unroll
   for (int i = 0; i < MAXTR; ++i) ftr_m[i] = 0;
-  T u0 = *I_(g.u, K, 0), v0 = *I_(g.v, K, 0), t0 = *I_(g.t, K, 0);
+  T u0 = *I_(g.u, K, k0), v0 = *I_(g.v, K, k0), t0 = *I_(g.t, K, k0);
   T tr0[MAXTR];
 #pragma unroll
-  for (int i = 0; i < MAXTR; ++i) tr0[i] = i < p.nt ? *I_(g.tr[i], K, 0) : (T)0;
-  T GP = 0;  // prefix sum_{1 <= h <= k} gp[h] td[h]
-  for (int k = 0; k < K; ++k) {
+  for (int i = 0; i < MAXTR; ++i) tr0[i] = i < p.nt ? *I_(g.tr[i], K, k0) : (T)0;
+  if (SPLIT && k0 > 0) {
+    const T c = cst[o.c2c + k0 - 1];
+    const T W = cst[o.ss + k0 - 1] * TF - PF;
+    fu_m = W * (u0 - *I_(g.u, K, k0 - 1)) * c;
+    fv_m = W * (v0 - *I_(g.v, K, k0 - 1)) * c;
+    ft_m = W * (t0 - *I_(g.t, K, k0 - 1)) * c;
+#pragma unroll
+    for (int i = 0; i < MAXTR; ++i)
+      if (i < p.nt) ftr_m[i] = W * (tr0[i] - *I_(g.tr[i], K, k0 - 1)) * c;
+    if (p.tnc) {
+      const T X = cst[o.ss + k0 - 1] * TE - PE;
+      fx_m = X * (cst[o.tref + k0] - cst[o.tref + k0 - 1]) * c;
+    }
+  }
+  for (int k = k0; k < k1; ++k) {
     const bool last = (k == K - 1);
     T u1 = 0, v1 = 0, t1 = 0, tr1[MAXTR];
 #pragma unroll
@@ -244,13 +304,13 @@ __global__ __launch_bounds__(256) void nodal_forward_kernel(
     T temp = t0 * d + (iva ? vadv_t : (T)0) + vadv_x + kappa * (mean_t + var_t);
     const T rt = R * t0 * adj;
     const T zt = z + fc;
-    *O_(g.cu, K, k) = -v0 * zt * s + ((iva ? -vadv_u : (T)0) + rt * gx) * s;
-    *O_(g.cv, K, k) = u0 * zt * s + ((iva ? -vadv_v : (T)0) + rt * gy) * s;
+    put(g.cu, K, k, -v0 * zt * s + ((iva ? -vadv_u : (T)0) + rt * gx) * s);
+    put(g.cv, K, k, u0 * zt * s + ((iva ? -vadv_v : (T)0) + rt * gy) * s);
     const T kinetic = (u0 * u0 + v0 * v0) * s / (T)2;
-    if (!moist) *O_(g.ke, K, k) = kinetic;
-    *O_(g.te, K, k) = temp;
-    *O_(g.ut, K, k) = u0 * t0 * s;
-    *O_(g.vt, K, k) = v0 * t0 * s;
+    if (!moist) put(g.ke, K, k, kinetic);
+    put(g.te, K, k, temp);
+    put(g.ut, K, k, u0 * t0 * s);
+    put(g.vt, K, k, v0 * t0 * s);
 #pragma unroll
     for (int i = 0; i < MAXTR; ++i) {
       if (i < p.nt) {
@@ -258,35 +318,31 @@ __global__ __launch_bounds__(256) void nodal_forward_kernel(
         T fx = W * (tr1[i] - x0) * c;
         T va = (T)-0.5 * (fx + ftr_m[i]);
         ftr_m[i] = fx;
-        *O_(g.trn[i], K, k) = (iva ? va : (T)0) + x0 * d;
-        *O_(g.tu[i], K, k) = u0 * x0 * s;
-        *O_(g.tv[i], K, k) = v0 * x0 * s;
+        put(g.trn[i], K, k, (iva ? va : (T)0) + x0 * d);
+        put(g.tu[i], K, k, u0 * x0 * s);
+        put(g.tv[i], K, k, v0 * x0 * s);
       }
     }
     if (moist) {
       T qx = *I_(g.qx, K, k), qy = *I_(g.qy, K, k);
       T cf = tref * (T)p.rvr;
-      *O_(g.curl, K, k) = cf * s * (gx * qy - gy * qx);
-      *O_(g.dc, K, k) = cf * s * (qx * gx + qy * gy) + q * lp * tref * (T)p.rvr;
+      put(g.curl, K, k, cf * s * (gx * qy - gy * qx));
+      put(g.dc, K, k, cf * s * (qx * gx + qy * gy) + q * lp * tref * (T)p.rvr);
       T td = q * (t0 + tref) * (T)p.gcr1;
       if (k >= 1) GP += cst[o.gp + k] * td;
-      *O_(g.ke, K, k) = kinetic + (cst[o.gd + k] * td + (GT - GP));
+      put(g.ke, K, k, kinetic + (cst[o.gd + k] * td + (GT - GP)));
     }
     fu_m = fu;
     fv_m = fv;
     ft_m = ft;
     PEm = PE;
     PFm = PF;
-    Wm = W;
-    Xm = X;
     u0 = u1;
     v0 = v1;
     t0 = t1;
 #pragma unroll
     for (int i = 0; i < MAXTR; ++i) tr0[i] = tr1[i];
   }
-  (void)Wm;
-  (void)Xm;
 }
 
 // ---------------------------------------------------------------- adjoint
@@ -642,9 +698,13 @@ int launch(bool adjoint, const dino_nodal* n, const void* in, const void* gout, 
   if constexpr (sizeof(T) == 8) cst = n->c64;
   else cst = n->c32;
   dim3 grid((unsigned)((p.IJ + 255) / 256), (unsigned)E);
-  if (!adjoint)
-    nodal_forward_kernel<T><<<grid, 256, 0, s>>>(static_cast<const T*>(in), static_cast<T*>(out),
-                                                 cst, g, p);
+  if (!adjoint && nodal_split(p.IJ * E))
+    nodal_forward_kernel<T, true><<<dim3((unsigned)((p.IJ + 63) / 64), (unsigned)E),
+                                    dim3(64, (unsigned)nodal_waves(p.K)), 0, s>>>(
+        static_cast<const T*>(in), static_cast<T*>(out), cst, g, p);
+  else if (!adjoint)
+    nodal_forward_kernel<T, false><<<grid, 256, 0, s>>>(static_cast<const T*>(in),
+                                                        static_cast<T*>(out), cst, g, p);
   else
     switch (n->nt) {
 #define ADJ_CASE(NTR)                                                                 \
