@@ -146,8 +146,8 @@ struct Params {
 // above and the flux through its top interface is formed from the level above.
 // Whole columns stream every field once, in order, at the copy rate, but a grid
 // of a few thousand columns is then a few dozen waves in a long chain: T42
-// L24, one member (8192 columns), 31 us whole and 16 split; T85 L24 moist, 2
-// members (65536), 73 and 46; TL255 L37 moist, one member (131072), 170 and 192.
+// L24, one member (8192 columns), 31 us whole and 17 split; T85 L24 moist, 2
+// members (65536), 71 and 48; TL255 L37 moist, one member (131072), 170 and 192.
 template <typename T, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_kernel(
     const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ cst, Groups g,

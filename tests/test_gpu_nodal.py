@@ -1,0 +1,58 @@
+"""Nodal kernel with a column's levels split over the waves of a block (small
+batches) and with whole columns (large ones) against the unfused formulation."""
+import numpy as np
+import pytest
+import torch
+
+from dinosaur_amd import coordinate_systems, primitive_equations as pe
+from dinosaur_amd import sigma_coordinates, spherical_harmonic as sh, units
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ('vorticity', 'divergence', 'temperature_variation', 'log_surface_pressure')
+CLOUDS = ('cloud_a', 'cloud_b')
+
+
+def _ragged():
+  # 200 columns: three blocks of 64 and one of 8
+  return sh.Grid(longitude_wavenumbers=7, total_wavenumbers=8, longitude_nodes=20,
+                 latitude_nodes=10)
+
+
+# Levels: one wave (1 to 3), an uneven share (5, 17, 37), the model's (12);
+# 12 and 13 members of T42 lie on both sides of the 98304 columns where the
+# whole-column kernel takes over.
+@pytest.mark.parametrize('grid,K,members,moist,tref_varies', [
+    (_ragged, 1, 1, False, False), (_ragged, 2, 3, True, True), (_ragged, 3, 1, False, True),
+    (_ragged, 5, 2, True, False), (_ragged, 17, 1, True, True), (_ragged, 37, 2, False, True),
+    (sh.Grid.T21, 12, 1, True, True), (sh.Grid.T42, 2, 12, True, True),
+    (sh.Grid.T42, 2, 13, True, True)])
+def test_split_and_whole_columns_match_unfused(grid, K, members, moist, tref_varies, gpu_device):
+  grid = grid()
+  coords = coordinate_systems.CoordinateSystem(
+      grid, sigma_coordinates.SigmaCoordinates.equidistant(K))
+  names = ['specific_humidity', *CLOUDS] if moist else ['passive']
+  kw = dict(humidity_key='specific_humidity', cloud_keys=CLOUDS) if moist else {}
+  tref = np.linspace(220., 290., K) if tref_varies else np.full(K, 250.0)
+  rs = np.random.RandomState(K + members)
+  l = grid.modal_mesh[1]
+
+  def field(lead, amp):
+    x = rs.normal(size=(members, lead) + grid.modal_shape) * grid.mask * amp / (l + 1) ** 1.5
+    return torch.as_tensor(x, device=gpu_device)
+
+  lnps = field(1, 0.05)
+  lnps[..., 0, 0] += 3.5449077 * 4.0
+  st = pe.State(field(K, 0.1), field(K, 0.1), field(K, 5.0), lnps,
+                tracers={n: field(K, 1e-3) for n in names})
+  oro = torch.as_tensor(rs.normal(size=grid.modal_shape) * grid.mask * 1e-4, device=gpu_device)
+  a, b = (pe.PrimitiveEquationsSigma(tref, oro, coords, units.SimUnits.from_si(),
+                                     fused_nodal=fused, **kw).explicit_terms(st)
+          for fused in (True, False))
+  pairs = [(f, getattr(a, f), getattr(b, f)) for f in FIELDS]
+  pairs += [(n, a.tracers[n], b.tracers[n]) for n in names]
+  for name, x, y in pairs:
+    # Only the order of sums differs: a few K eps = 1e-14 of the largest terms, which
+    # the divergence's Laplacian leaves up to 1e2 times larger than their sum.
+    err = (x - y).abs().max().item() / max(y.abs().max().item(), 1e-300)
+    assert err < 1e-12, (name, err)
