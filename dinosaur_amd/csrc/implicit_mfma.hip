@@ -31,14 +31,25 @@
 #include "dino_common.h"
 
 namespace dino {
+
+int device_cus();  // dft.hip
+
 namespace {
 
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWavesPerBlock = 8;  // waves sharing one LDS copy of the tables
-// 16-column tiles each wave processes: the block's copy of the tables (tens
-// of KiB from L2) then serves kRepeats x 8 tiles instead of 8
-constexpr int kRepeats = 4;
+// 16-column tiles each wave processes, one after the other.  Two share the
+// block's copy of the tables (tens of KiB from L2) where the launch fills the
+// chip; up to 8 blocks per CU the second tile only lengthens the chain (table
+// copy, loads, FP64 MFMAs, stores) of a chip with idle waves.  Solve, FP32, one /
+// two tiles a wave: T21 L12 (62 tiles) 5.0 / 7.2 us, TL127 L32 (2056) 15.6 / 20.1,
+// TL127 L32, 4 members (8224) 34.1 / 34.7, 8 members (16448) 60.0 / 61.3, TL255 L37,
+// 4 members (32832) 145 / 129, 16 members (131328) 539 / 474; four: 11.7, 35.0,
+// 49.1, 63.4, 139, 479.
+inline int tiles_per_wave(int64_t tiles) {
+  return tiles <= (int64_t)8 * kWavesPerBlock * device_cus() ? 1 : 2;
+}
 
 __device__ __forceinline__ doublex4 mma64(double a, double b, doublex4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
@@ -106,7 +117,8 @@ void solve_mfma_kernel(
     const double* __restrict__ t1a_g, const double* __restrict__ t1b_g,
     const double* __restrict__ t2_g, const double* __restrict__ wvec,
     const double* __restrict__ dvec, const double* __restrict__ lam, int K, int L,
-    int64_t cols, int64_t members, double eta, int tri, int inplace) {
+    int64_t cols, int64_t members, double eta, int tri, int inplace,
+    int repeats) {
   constexpr bool ACCUM = false;
   using S = Shape<NS>;
   // the block's waves share the operand tables through LDS (one L2 read per
@@ -221,10 +233,10 @@ void solve_mfma_kernel(
   // the lnps row lives in one k-group
   if (kg == (lrow & 3) && cok) lnps_out[(int64_t)b * cols + cc] = (T)(lp - c2 * sacc);
   };
-  const int first = (int)blockIdx.x * kRepeats * kWavesPerBlock + (int)(threadIdx.x >> 6);
+  const int first = (int)blockIdx.x * repeats * kWavesPerBlock + (int)(threadIdx.x >> 6);
   const int n_waves = tiles_per_member * (int)members;
 #pragma unroll 1
-  for (int rep = 0; rep < kRepeats; ++rep) {
+  for (int rep = 0; rep < repeats; ++rep) {
     const int wave = first + rep * kWavesPerBlock;
     if (wave >= n_waves) break;
     // an opaque copy of the lane index keeps the table reads inside the loop
@@ -246,7 +258,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void terms_mfma_kernel(
     const T* div, const T* temp, const T* lnps, T* div_out, T* temp_out, T* lnps_out,
     const double* __restrict__ tg_g, const double* __restrict__ th_g,
     const double* __restrict__ rtref, const double* __restrict__ lam, int K, int L,
-    int64_t cols, int64_t members, int tri, int inplace) {
+    int64_t cols, int64_t members, int tri, int inplace, int repeats) {
   constexpr bool ACCUM = ACC;  // adding the zero result changes nothing
   using S = Shape<NS>;
   constexpr int NG = S::T1 * NS * 64, NH = S::TT * NS * 64;
@@ -336,10 +348,10 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void terms_mfma_kernel(
     *o = ACC ? (T)(*o + v) : v;
   }
   };
-  const int first = (int)blockIdx.x * kRepeats * kWavesPerBlock + (int)(threadIdx.x >> 6);
+  const int first = (int)blockIdx.x * repeats * kWavesPerBlock + (int)(threadIdx.x >> 6);
   const int n_waves = tiles_per_member * (int)members;
 #pragma unroll 1
-  for (int rep = 0; rep < kRepeats; ++rep) {
+  for (int rep = 0; rep < repeats; ++rep) {
     const int wave = first + rep * kWavesPerBlock;
     if (wave >= n_waves) break;
     // an opaque copy of the lane index keeps the table reads inside the loop
@@ -450,10 +462,11 @@ static int launch_ns(bool solve, bool adjoint, bool acc, const dino_implicit* f,
   const int64_t waves = (cols + 15) / 16 * members;
   if (waves == 0) return DINO_OK;
   // column tiles and columns are indexed with 32-bit integers in the kernels
-  DINO_REQUIRE(waves + (int64_t)kWavesPerBlock * kRepeats < ((int64_t)1 << 31) &&
+  DINO_REQUIRE(waves + (int64_t)kWavesPerBlock * 4 < ((int64_t)1 << 31) &&
                    cols < ((int64_t)1 << 31),
                DINO_EINVAL, "implicit solve: too many columns for one launch");
-  const int64_t per_block = (int64_t)kWavesPerBlock * kRepeats;
+  const int repeats = tiles_per_wave(waves);
+  const int64_t per_block = (int64_t)kWavesPerBlock * repeats;
   const unsigned blocks = (unsigned)((waves + per_block - 1) / per_block);
   const unsigned threads = 64 * kWavesPerBlock;
   const T* x0 = (const T*)div;
@@ -468,23 +481,23 @@ static int launch_ns(bool solve, bool adjoint, bool acc, const dino_implicit* f,
   if (solve && !adjoint) {
     solve_mfma_kernel<T, NS, false><<<blocks, threads, 0, s>>>(
         x0, x1, x2, y0, y1, y2, t[0], t[1], t[2], t[3], t[4], f->lam, f->K, f->L, cols,
-        members, f->eta, tri, inplace);
+        members, f->eta, tri, inplace, repeats);
   } else if (solve) {
     solve_mfma_kernel<T, NS, true><<<blocks, threads, 0, s>>>(
         x0, x1, x2, y0, y1, y2, t[8], t[9], t[10], t[11], t[4], f->lam, f->K, f->L, cols,
-        members, f->eta, tri, inplace);
+        members, f->eta, tri, inplace, repeats);
   } else if (!adjoint) {
     terms_mfma_kernel<T, NS, false, false><<<blocks, threads, 0, s>>>(
         x0, x1, x2, y0, y1, y2, t[5], t[6], t[7], f->lam, f->K, f->L, cols, members, tri,
-        inplace);
+        inplace, repeats);
   } else if (!acc) {
     terms_mfma_kernel<T, NS, true, false><<<blocks, threads, 0, s>>>(
         x0, x1, x2, y0, y1, y2, t[12], t[13], t[14], f->lam, f->K, f->L, cols, members, tri,
-        inplace);
+        inplace, repeats);
   } else {
     terms_mfma_kernel<T, NS, true, true><<<blocks, threads, 0, s>>>(
         x0, x1, x2, y0, y1, y2, t[12], t[13], t[14], f->lam, f->K, f->L, cols, members, tri,
-        inplace);
+        inplace, repeats);
   }
   DINO_LAUNCH_CHECK("implicit mfma kernel");
   return DINO_OK;
