@@ -23,6 +23,7 @@
 // UP2 = (l-1) a_lm, DN2 = -(l+2) b_lm (sec_lat_d_dlat_cos2, :1085-1092).
 // dlon is antisymmetric; the adjoints of cldl/sdlc are the transposed
 // two-point stencils.  One thread per (member, r, l) walks a chunk of levels.
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -128,13 +129,17 @@ struct MP {
   double a, g;
 };
 
-// Levels one thread walks: chunks of 4 levels give the launch ~9x more
-// threads than whole columns at 37 levels, and 10-18% shorter kernels at
-// TL255 x 16 members (more loads in flight; the per-position stencil
-// coefficients are re-read per chunk, from cache).
-#ifndef DINO_MODAL_LEVELS_PER_THREAD
-#define DINO_MODAL_LEVELS_PER_THREAD 4
-#endif
+// Levels one thread walks.  More of them share a position's stencil
+// coefficients, fewer put more loads in flight and shorten the chain of a
+// launch that does not fill the chip.  Prep / epilogue with 1, 2 and 4 levels
+// a thread (us): T21 L12 3.8, 4.3, 5.3 / 3.6, 4.2, 5.2; T42 L24 moist (9e4 entries)
+// 4.9, 5.8, 8.2 / 5.2, 6.3, 9.3; T85 L24 moist (3.6e5) 7.0, 7.6, 9.5 / 9.7, 9.9, 13.7;
+// T42 L24, 4 members (3.6e5) 5.8, 5.7, 6.2 / 6.2, 5.5, 6.1; TL255 L37 moist (4.9e6)
+// 44, 39, 42 / 83, 79, 83, 16 members (7.8e7) 996, 985, 983 / 1225, 1158, 1144, their
+// adjoints 1104, 1009, 995 / 1509, 1525, 1545.
+inline int levels_per_thread(int64_t entries) {
+  return entries <= (1 << 18) ? 1 : entries <= (1 << 25) ? 2 : 4;
+}
 
 // Stencil of one thread's (r, l): the bidiagonal-in-l operators read the
 // neighbours l - 1 and l + 1.  Out-of-range neighbours are loaded from a
@@ -508,7 +513,7 @@ const T* consts(const dino_modal* m) {
   else return m->c32;
 }
 
-MP make_mp(const dino_modal* m) {
+MP make_mp(const dino_modal* m, int64_t E) {
   MP p;
   p.R = m->R;
   p.L = m->L;
@@ -517,9 +522,9 @@ MP make_mp(const dino_modal* m) {
   p.hum = m->hybrid ? -1 : m->hum;
   p.lnps = m->hybrid || m->forced;
   p.forced = m->forced;
-  p.kc = DINO_MODAL_LEVELS_PER_THREAD < m->K ? DINO_MODAL_LEVELS_PER_THREAD : m->K;
-  p.nkc = (m->K + p.kc - 1) / p.kc;
   p.RL = (int64_t)m->R * m->L;
+  p.kc = std::min(levels_per_thread(p.RL * m->K * E), m->K);
+  p.nkc = (m->K + p.kc - 1) / p.kc;
   p.a = m->radius;
   p.g = m->gravity;
   return p;
@@ -528,7 +533,7 @@ MP make_mp(const dino_modal* m) {
 template <typename T>
 int run(int which, const dino_modal* m, const void* a, const void* b, void* out, int64_t E,
         hipStream_t s) {
-  MP p = make_mp(m);
+  MP p = make_mp(m, E);
   // level chunks: as many as the grid's y extent allows for E members
   while ((int64_t)p.nkc * E > 65535) {
     p.kc *= 2;
@@ -565,7 +570,7 @@ int run(int which, const dino_modal* m, const void* a, const void* b, void* out,
 template <typename T>
 int run_winds(int mode, const dino_modal* m, const void* x0, const void* x1, void* y0, void* y1,
               int64_t B, int clip, hipStream_t s) {
-  const MP p = make_mp(m);
+  const MP p = make_mp(m, 1);
   int64_t per = 4;  // fields per thread, as the levels of the other modal kernels
   while ((B + per - 1) / per > 65535) per *= 2;
   const bool tiles = mode == 0 || mode == 3;  // outputs the inverse transform reads
