@@ -411,7 +411,7 @@ __global__ __launch_bounds__(64 * NW, (fwd_waves_per_simd<NW, KS>())) void leg_f
 // did not fit), and both fill the strip's output ring.  NS strips (16 NS rows)
 // per workgroup: the table of a large grid (262 MB at TL639) is the largest
 // operand at common batches, so a workgroup takes as many rows of one m as
-// there are, up to 128.  kt of the KT node groups are in use.
+// there are, up to 128.  2 ks of the KT node groups are in use, a half in each chain.
 // TL639, 37 fields: 519 us with the tiled kernel, 223 us here (table and rows
 // 0.08 ms at the copy rate, 10.6 GFLOP of tiles 0.07 ms).
 template <int KT, int NS, bool VIN>
@@ -424,7 +424,8 @@ __global__ __launch_bounds__(128 * NS) void leg_fwd_split_rows_kernel(
   constexpr int PER = (128 * KT + NTH - 1) / NTH;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   floatx4* const lds = reinterpret_cast<floatx4*>(smem_raw);
-  const int tf4 = tile_f4(ks), kt = 2 * ks;
+  constexpr int KH = KT / 2;
+  const int tf4 = tile_f4(ks);
   const int m = m_of_block(blockIdx.y, gridDim.y, mpair);
   const int nrows = (m == 0) ? B : 2 * B;
   const int row0 = blockIdx.x * RPB;
@@ -463,16 +464,17 @@ __global__ __launch_bounds__(128 * NS) void leg_fwd_split_rows_kernel(
     const float *const up = f + J - Jh + j0, *const down = f + Jh - 4 - j0;
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
-      const int jj = 16 * t + 4 * g;
+      // slots [0, ks) and [KH, KH + ks) hold the two halves of the 2 ks groups
+      const int q0 = 16 * (t < KH ? t : t - KH + ks), jj = q0 + 4 * g;
       x[t] = zero;
-      if (16 * t >= Jh) continue;
+      if (t % KH >= ks || q0 >= Jh) continue;
       if constexpr (VIN) {
-        // whole groups at constant offsets from two row pointers; the last one
-        // may be partial (Jh % 4 == 0: whole vectors)
-        const bool in = 16 * t + 16 <= Jh || jj < Jh;
-        const int off = in ? 16 * t : 0;
-        const floatx4 u = *reinterpret_cast<const floatx4*>(up + off);
-        const floatx4 dr = *reinterpret_cast<const floatx4*>(down - off);
+        // whole groups at constant offsets from two row pointers for each half;
+        // the last one may be partial (Jh % 4 == 0: whole vectors)
+        const bool in = q0 + 16 <= Jh || jj < Jh;
+        const int half = t < KH ? 0 : 16 * (ks - KH), off = in ? 16 * t : -half;
+        const floatx4 u = *reinterpret_cast<const floatx4*>(up + half + off);
+        const floatx4 dr = *reinterpret_cast<const floatx4*>(down - half - off);
         const floatx4 v = u + sgn * floatx4{dr[3], dr[2], dr[1], dr[0]};
         x[t] = rok && in ? v : zero;
       } else {
@@ -535,20 +537,24 @@ __global__ __launch_bounds__(128 * NS) void leg_fwd_split_rows_kernel(
     __builtin_amdgcn_sched_barrier(0);
     const int lt = lt0 + tt * kTileDeg;
     if (used) {
-      // two accumulator chains (even and odd groups), so that the matrix core
-      // need not wait for the previous product
+      // two accumulator chains, so that the matrix core need not wait for the
+      // previous product: one for each contiguous half of the nodes.  Partial sums
+      // over neighbouring nodes stay small where the whole sum does; chains of
+      // alternate groups would not be orthogonal by themselves (they alias at the
+      // degrees of the groups' period, l = 40 of TL639) and lose there what the
+      // final sum cancels: 5 times the error of m = 0 and 1.
       floatx4 a0 = zero, a1 = zero;
 #pragma unroll
-      for (int t = 0; t < KT; t += 2) {
-        if (t >= kt) continue;  // kt is even
+      for (int t = 0; t < KH; ++t) {
+        if (t >= ks) continue;
         // reads a tile's table a few groups ahead, not all of it (registers)
-        if (t % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-        const floatx4 p0 = buf[(par * kt + t) * 64 + lane];
-        const floatx4 p1 = buf[(par * kt + t + 1) * 64 + lane];
+        if (t % 2 == 0) __builtin_amdgcn_sched_barrier(0);
+        const floatx4 p0 = buf[(par * 2 * ks + t) * 64 + lane];
+        const floatx4 p1 = buf[(par * 2 * ks + ks + t) * 64 + lane];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[t][u], p0[u], a0, 0, 0, 0);
-          a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[t + 1][u], p1[u], a1, 0, 0, 0);
+          a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(x[KH + t][u], p1[u], a1, 0, 0, 0);
         }
       }
       // degrees lt + 2 c16 + par of rows 4 g + i
