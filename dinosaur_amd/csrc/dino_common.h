@@ -128,6 +128,24 @@ __device__ __forceinline__ int m_of_block(int y, int M, int paired) {
   return paired ? ((y & 1) ? M - 1 - (y >> 1) : (y >> 1)) : y;
 }
 
+// Launch order of the row-resident Legendre kernels: bit 0 pairs short and long m,
+// bit 1 is the XCD order below (grid y then padded to a multiple of 8, and a block
+// whose y is M or more has no work).
+constexpr int kOrderPaired = 1, kOrderXcd = 2;
+
+// Consecutive workgroups go to the 8 XCDs in turn.  In XCD order the row blocks of
+// one m, which read the same Legendre table, follow each other on one XCD, so its L2
+// serves the table to all but the first.
+__device__ __forceinline__ void row_block(int order, int* x, int* y) {
+  *x = blockIdx.x;
+  *y = blockIdx.y;
+  if (order & kOrderXcd) {
+    const int nx = gridDim.x, id = *x + nx * *y, slot = id >> 3;
+    *y = (slot / nx) * 8 + (id & 7);
+    *x = slot % nx;
+  }
+}
+
 struct dino_implicit {
   int K, L, R;
   double r_gas, eta;

@@ -6,7 +6,7 @@
 //
 // Like the forward kernel (legendre_rows.hip) this is HBM-bound, so the
 // layout reads the modal rows once and writes the Fourier rows once:
-//   * a workgroup owns 64 rows (4 waves x 16) of one zonal wavenumber m and
+//   * a workgroup owns 64 rows (strips of 16; some launches 96) of one m and
 //     keeps the accumulators of every node tile in VGPRs while it sweeps the
 //     32-degree tiles of that m;
 //   * per tile, each row of the workgroup brings in one whole 128-byte line
@@ -18,7 +18,7 @@
 //   * at the end the up / down halves are staged in LDS and written as whole
 //     contiguous row segments;
 //   * above 128 northern nodes the nodes are split into even blocks, one
-//     workgroup each (TL639, 37 fields: 367 us with the tiled kernel, 228 here,
+//     workgroup each (TL639, 37 fields: 367 us with the tiled kernel, 166 here,
 //     its table of 330 MB being the largest operand).  Node tiles come in 1, 2,
 //     4, 6 or 8 per block (80 or 90 nodes take 6, not 8).
 //
@@ -35,7 +35,6 @@ namespace {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 
-constexpr int kRows = 64;
 constexpr int kTile = 32;
 constexpr int kRingPitch = 68;  // modal ring row pitch (floats): 64 degrees + 4
 
@@ -70,20 +69,22 @@ __device__ __forceinline__ float bf16_value(unsigned short h) {
 // per CU to overlap the MFMAs with the loads and stores of other waves (the
 // FP32 register budget of 6 waves per SIMD lets 3 such blocks share a CU;
 // the split path would spill under it).
+// SP: strips of 16 rows per block.
 // BLK: the nodes are split into blocks (Jh > 128) of int_block nodes, one per z.
-template <bool BF, int NT, bool VOUT, int WS, bool BLK>
-__global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows_kernel(
+template <bool BF, int NT, bool VOUT, int WS, bool BLK, int SP>
+__global__ __launch_bounds__(64 * SP * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows_kernel(
     const float* __restrict__ modal, float* __restrict__ fourier,
     const float4* __restrict__ itab, const int64_t* __restrict__ itile_off, int B, int L,
-    int J, int Jh, int Rrows, int mpair, int block_nodes) {
+    int J, int Jh, int Rrows, int order, int block_nodes) {
   static_assert(NT % WS == 0, "the waves of a strip split the node tiles evenly");
-  constexpr int NTH = 256 * WS;  // threads
+  constexpr int NTH = 64 * SP * WS;  // threads
+  constexpr int kRows = 16 * SP;     // rows
   constexpr int NTW = NT / WS;   // node tiles per wave
   constexpr int RPL = 2 / WS;    // modal line quads per lane per tile
   constexpr int TF4 = inv_tile_f4(NT);
   constexpr int PER = (TF4 + NTH - 1) / NTH;
   constexpr int OPITCH = 16 * NT + 4;
-  constexpr int OUT4 = 4 * 16 * OPITCH / 4;
+  constexpr int OUT4 = SP * 16 * OPITCH / 4;
   constexpr int MAIN4 = (2 * TF4 > OUT4) ? 2 * TF4 : OUT4;
   __shared__ floatx4 lds[MAIN4];
   // Modal rows arrive as whole 128-byte lines (float4 loads, one new line
@@ -93,14 +94,18 @@ __global__ __launch_bounds__(256 * WS, WS == 2 && !BF ? 6 : 1) void leg_inv_rows
   // hold it.  A TL row holds an odd number of degrees, so tile-sized
   // segments would start anywhere in a line and split into partial
   // requests.
-  __shared__ floatx4 ring4[4 * 16 * kRingPitch / 4];
+  __shared__ floatx4 ring4[SP * 16 * kRingPitch / 4];
   float* const ring = reinterpret_cast<float*>(ring4);
-  const int m = m_of_block(blockIdx.y, gridDim.y, mpair);
+  int bx, by;
+  row_block(order, &bx, &by);
+  const int M = (Rrows + 1) / 2;
+  if (by >= M) return;
+  const int m = m_of_block(by, M, order & kOrderPaired);
   const int nrows = (m == 0) ? B : 2 * B;
-  const int row0 = blockIdx.x * kRows;
+  const int row0 = bx * kRows;
   if (row0 >= nrows) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int strip = wave & 3, wh = wave >> 2;  // wh: this wave's share of the strip
+  const int strip = wave % SP, wh = wave / SP;  // wh: this wave's share of the strip
   const int g = lane >> 4, c16 = lane & 15;
   const int lt0 = leg_tile_start(m, L);
   const int ntile = inv_tiles_of_m(m, L);
@@ -346,32 +351,59 @@ __global__ void inverse_fragments_kernel(int L, int Jh, int Jhp, int NT, int NB,
   w[3] = lo[2] | ((uint32_t)lo[3] << 16);
 }
 
-template <bool BF, int NT>
-int launch_inv_rows(const dino_plan* pl, const float* in, float* out, int64_t B, hipStream_t s) {
+// XCD order (row_block) where it pays, us without and with it: T106 111 fields 14.5 /
+// 13.8, TL255 37 26.1 / 25.1, 222 69.6 / 67.0, 400 110.5 / 110.4, T213 200 72.3 / 67.9,
+// TL639 100 421 / 401; not up to 64 nodes (T85 1000 39.6 / 40.2: the table is small)
+// nor, in FP32, for many row blocks of up to 128 nodes (TL255 1000 256 / 259, 2400
+// 587 / 601: bound by the rows, whose neighbours in m then lie on different XCDs;
+// split BF16 gains there too, 512 / 507).
+inline bool inverse_xcd_order(int Jh, int64_t row_blocks, bool bf) {
+  return Jh > 128 || (Jh > 64 && (bf || row_blocks <= 14));
+}
+
+// 96 rows per workgroup where they make one of two: the table is read once.  Pays
+// when it does not stay in the L2s (32 MB): 37 fields of TL639 209 us with 64 rows, 166
+// here, T340 62 and 46, but T213 (15 MB) 22.3 and 23.9; 100 fields of TL639 (three
+// workgroups for four) 401 and 406.
+inline bool inverse_wide_rows(const dino_plan* pl, int64_t B) {
+  return B > 32 && B <= 48 && (int64_t)pl->M * pl->L * pl->Jh * 2 > (int64_t)32 << 20;
+}
+
+template <bool BF, int NT, bool BK, int SP>
+int launch_strips(const dino_plan* pl, const float* in, float* out, int64_t B, hipStream_t s) {
+  constexpr int kRows = 16 * SP;
   const bool vout = pl->J % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-  const dim3 grid((unsigned)((2 * B + kRows - 1) / kRows), (unsigned)pl->M, (unsigned)pl->int_nb);
+  const int64_t gx = (2 * B + kRows - 1) / kRows;
+  const bool xcd = inverse_xcd_order(pl->Jh, gx, BF);
+  const dim3 grid((unsigned)gx, (unsigned)(xcd ? (pl->M + 7) / 8 * 8 : pl->M),
+                  (unsigned)pl->int_nb);
   const float4* tab = BF ? reinterpret_cast<const float4*>(pl->ifragbf)
                          : reinterpret_cast<const float4*>(pl->ifrag32);
-  const int mpair = (pl->sched[DINO_STAGE_LEGENDRE_INVERSE] & DINO_SCHED_MPAIRED) ? 1 : 0;
+  const int order = ((pl->sched[DINO_STAGE_LEGENDRE_INVERSE] & DINO_SCHED_MPAIRED) ? kOrderPaired : 0) |
+                    (xcd ? kOrderXcd : 0);
   // two waves per strip whenever the node tiles split evenly
   constexpr int WS = NT % 2 == 0 ? 2 : 1;
-#define INV_LAUNCH(VO, BK)                                                             \
-  leg_inv_rows_kernel<BF, NT, VO, WS, BK><<<grid, 256 * WS, 0, s>>>(                    \
-      in, out, tab, pl->itile_off, (int)B, pl->L, pl->J, pl->Jh, pl->R, mpair, pl->int_block)
-  // blocks of at least 65 nodes: only the 6- and 8-tile forms
-  if constexpr (NT >= 6) {
-    if (pl->int_nb > 1) {
-      if (vout) INV_LAUNCH(true, true);
-      else INV_LAUNCH(false, true);
-      DINO_LAUNCH_CHECK("legendre inverse rows kernel");
-      return DINO_OK;
-    }
-  }
-  if (vout) INV_LAUNCH(true, false);
-  else INV_LAUNCH(false, false);
+#define INV_LAUNCH(VO)                                                                     \
+  leg_inv_rows_kernel<BF, NT, VO, WS, BK, SP><<<grid, 64 * SP * WS, 0, s>>>(                \
+      in, out, tab, pl->itile_off, (int)B, pl->L, pl->J, pl->Jh, pl->R, order, pl->int_block)
+  if (vout) INV_LAUNCH(true);
+  else INV_LAUNCH(false);
 #undef INV_LAUNCH
   DINO_LAUNCH_CHECK("legendre inverse rows kernel");
   return DINO_OK;
+}
+
+template <bool BF, int NT>
+int launch_inv_rows(const dino_plan* pl, const float* in, float* out, int64_t B, hipStream_t s) {
+  // node blocks hold at least 65 nodes: only the 6- and 8-tile forms
+  if constexpr (NT >= 6) {
+    if (pl->int_nb > 1) {
+      if constexpr (!BF)
+        if (inverse_wide_rows(pl, B)) return launch_strips<BF, NT, true, 6>(pl, in, out, B, s);
+      return launch_strips<BF, NT, true, 4>(pl, in, out, B, s);
+    }
+  }
+  return launch_strips<BF, NT, false, 4>(pl, in, out, B, s);
 }
 
 template <bool BF>
@@ -424,9 +456,10 @@ void inverse_fragment_fill(const dino_plan* pl, hipStream_t s) {
 int legendre_inverse_rows(const dino_plan* pl, const float* in, float* out, int64_t B,
                           bool split, hipStream_t s) {
   if (B == 0) return DINO_OK;
-  DINO_REQUIRE(2 * B / kRows < (int64_t)1 << 30, DINO_EINVAL, "batch too large");
-  // a block's modal rows span at most 64 fields, addressed with 32-bit offsets
-  DINO_REQUIRE((int64_t)kRows * pl->R * pl->L < (int64_t)1 << 31, DINO_EINVAL,
+  DINO_REQUIRE(2 * B / 64 < (int64_t)1 << 30, DINO_EINVAL, "batch too large");
+  // a block's modal rows span at most 64 fields (48 where it has 96 rows, as B
+  // is no larger), addressed with 32-bit offsets
+  DINO_REQUIRE((int64_t)64 * pl->R * pl->L < (int64_t)1 << 31, DINO_EINVAL,
                "modal fields too large for the row kernel");
   return split ? inv_rows_by_nt<true>(pl, in, out, B, s) : inv_rows_by_nt<false>(pl, in, out, B, s);
 }

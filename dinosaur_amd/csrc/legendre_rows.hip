@@ -138,7 +138,7 @@ template <bool BF, int KS, bool VIN, int NW>
 __global__ __launch_bounds__(64 * NW, (fwd_waves_per_simd<NW, KS>())) void leg_fwd_rows_kernel(
     const float* __restrict__ fourier, float* __restrict__ modal,
     const float4* __restrict__ ftab, const int64_t* __restrict__ ftile_off,
-    float* __restrict__ sink, int B, int L, int J, int Jh, int Rrows, int mpair, int skip_zero) {
+    float* __restrict__ sink, int B, int L, int J, int Jh, int Rrows, int order, int skip_zero) {
   constexpr int KT = 2 * KS;  // 16-node groups
   constexpr int NTH = 64 * NW;  // threads
   constexpr int RPB = kRowsPerWave * NW;  // rows per workgroup
@@ -153,9 +153,13 @@ __global__ __launch_bounds__(64 * NW, (fwd_waves_per_simd<NW, KS>())) void leg_f
   constexpr int LDS4 = (2 * TF4 + RING4 > STG4) ? 2 * TF4 + RING4 : STG4;
   __shared__ floatx4 lds[LDS4];
   float* const ring = reinterpret_cast<float*>(lds + 2 * TF4);
-  const int m = m_of_block(blockIdx.y, gridDim.y, mpair);
+  int bx, by;
+  row_block(order, &bx, &by);
+  const int M = (Rrows + 1) / 2;
+  if (by >= M) return;
+  const int m = m_of_block(by, M, order & kOrderPaired);
   const int nrows = (m == 0) ? B : 2 * B;
-  const int row0 = blockIdx.x * RPB;
+  const int row0 = bx * RPB;
   if (row0 >= nrows) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, c16 = lane & 15;
@@ -418,7 +422,7 @@ template <int KT, int NS, bool VIN>
 __global__ __launch_bounds__(128 * NS) void leg_fwd_split_rows_kernel(
     const float* __restrict__ fourier, float* __restrict__ modal,
     const float4* __restrict__ ftab, const int64_t* __restrict__ ftile_off,
-    float* __restrict__ sink, int B, int L, int J, int Jh, int Rrows, int ks, int mpair,
+    float* __restrict__ sink, int B, int L, int J, int Jh, int Rrows, int ks, int order,
     int skip_zero) {
   constexpr int NTH = 128 * NS, RPB = 16 * NS;
   constexpr int PER = (128 * KT + NTH - 1) / NTH;
@@ -426,9 +430,13 @@ __global__ __launch_bounds__(128 * NS) void leg_fwd_split_rows_kernel(
   floatx4* const lds = reinterpret_cast<floatx4*>(smem_raw);
   constexpr int KH = KT / 2;
   const int tf4 = tile_f4(ks);
-  const int m = m_of_block(blockIdx.y, gridDim.y, mpair);
+  int bx, by;
+  row_block(order, &bx, &by);
+  const int M = (Rrows + 1) / 2;
+  if (by >= M) return;
+  const int m = m_of_block(by, M, order & kOrderPaired);
   const int nrows = (m == 0) ? B : 2 * B;
-  const int row0 = blockIdx.x * RPB;
+  const int row0 = bx * RPB;
   if (row0 >= nrows) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int strip = wave >> 1, par = wave & 1;  // the wave's strip and fold parity
@@ -630,18 +638,26 @@ __global__ void forward_fragments_kernel(int L, int Jh, int Jhp, int ks,
   }
 }
 
+// XCD order (row_block) above 64 nodes, us without and with it: T106 111 fields 13.7 /
+// 13.3, TL179 100 28.6 / 27.8, TL255 222 74.9 / 73.8, 2400 646 / 639, TL639 100 474 /
+// 463, 200 937 / 901 (split BF16: T213 200 53.9 / 51.7); up to 64 nodes the table is
+// small (T85 96 9.3 / 9.5, 1000 41.1 / 41.9).
+inline bool forward_xcd_order(int Jh) { return Jh > 64; }
+
 template <bool BF, int KS, int NW>
 int launch_rows(const dino_plan* pl, const float* in, float* out, int64_t B, int skip_zero,
                 hipStream_t s) {
   constexpr int RPB = kRowsPerWave * NW;
   const bool vin = pl->J % 8 == 0 && reinterpret_cast<uintptr_t>(in) % 16 == 0;
-  const dim3 grid((unsigned)((2 * B + RPB - 1) / RPB), (unsigned)pl->M);
+  const bool xcd = forward_xcd_order(pl->Jh);
+  const dim3 grid((unsigned)((2 * B + RPB - 1) / RPB), (unsigned)(xcd ? (pl->M + 7) / 8 * 8 : pl->M));
   const float4* tab = BF ? reinterpret_cast<const float4*>(pl->ffragbf)
                          : reinterpret_cast<const float4*>(pl->ffrag32);
-  const int mpair = (pl->sched[DINO_STAGE_LEGENDRE_FORWARD] & DINO_SCHED_MPAIRED) ? 1 : 0;
+  const int order = ((pl->sched[DINO_STAGE_LEGENDRE_FORWARD] & DINO_SCHED_MPAIRED) ? kOrderPaired : 0) |
+                    (xcd ? kOrderXcd : 0);
 #define ROWS_LAUNCH(VI)                                                                   \
   leg_fwd_rows_kernel<BF, KS, VI, NW><<<grid, 64 * NW, 0, s>>>(                            \
-      in, out, tab, pl->ftile_off, pl->sink, (int)B, pl->L, pl->J, pl->Jh, pl->R, mpair,  \
+      in, out, tab, pl->ftile_off, pl->sink, (int)B, pl->L, pl->J, pl->Jh, pl->R, order,  \
       skip_zero)
   if (vin) ROWS_LAUNCH(true);
   else ROWS_LAUNCH(false);
@@ -677,8 +693,10 @@ template <int KT, int NS>
 int launch_split_rows(const dino_plan* pl, const float* in, float* out, int64_t B, int skip_zero,
                       hipStream_t s) {
   const bool vin = pl->J % 8 == 0 && reinterpret_cast<uintptr_t>(in) % 16 == 0;
-  const dim3 grid((unsigned)((2 * B + 16 * NS - 1) / (16 * NS)), (unsigned)pl->M);
-  const int mpair = (pl->sched[DINO_STAGE_LEGENDRE_FORWARD] & DINO_SCHED_MPAIRED) ? 1 : 0;
+  const bool xcd = forward_xcd_order(pl->Jh);
+  const dim3 grid((unsigned)((2 * B + 16 * NS - 1) / (16 * NS)), (unsigned)(xcd ? (pl->M + 7) / 8 * 8 : pl->M));
+  const int order = ((pl->sched[DINO_STAGE_LEGENDRE_FORWARD] & DINO_SCHED_MPAIRED) ? kOrderPaired : 0) |
+                    (xcd ? kOrderXcd : 0);
   const size_t lds = 16 * (size_t)(2 * tile_f4(pl->fks)) + 4 * (size_t)(16 * NS * kRingPitch);
   const float4* tab = reinterpret_cast<const float4*>(pl->ffrag32);
 #define SPLIT_LAUNCH(VI)                                                                      \
@@ -687,7 +705,7 @@ int launch_split_rows(const dino_plan* pl, const float* in, float* out, int64_t 
     DINO_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));   \
     leg_fwd_split_rows_kernel<KT, NS, VI><<<grid, 128 * NS, lds, s>>>(                         \
         in, out, tab, pl->ftile_off, pl->sink, (int)B, pl->L, pl->J, pl->Jh, pl->R, pl->fks,  \
-        mpair, skip_zero);                                                                    \
+        order, skip_zero);                                                                    \
   } while (0)
   if (vin) SPLIT_LAUNCH(true);
   else SPLIT_LAUNCH(false);
