@@ -12,13 +12,15 @@
 // (spherical_harmonic.py:265, 277-279), which multiply by the l < m zeros and
 // the duplicated +/-m rows of the reference's (2M-1, J, L) table.
 //
-// This file holds the plain FMA kernels (FP32 or FP64 arithmetic); the split
-// FP16/BF16 MFMA kernels live in legendre_mfma.hip.
+// This file holds the plain FP64 FMA kernels, which serve the sizes where the FP64
+// matrix-core kernels (legendre_f64.hip) are slower; FP32 data takes legendre_rows.hip,
+// legendre_inv_rows.hip and legendre_mfma.hip.
 #include "dino_common.h"
 
 namespace dino {
 namespace {
 
+using T = double;
 constexpr int TR = 64;   // rows (fields x cos/sin) per tile
 constexpr int TC = 64;   // latitudes (inverse) or degrees (forward) per tile
 constexpr int KC = 16;   // contraction chunk
@@ -34,7 +36,6 @@ __device__ __forceinline__ void row_of(int m, int q, int* b, int* r) {
   }
 }
 
-template <typename T>
 __global__ __launch_bounds__(NT) void legendre_inverse_fma_kernel(
     const T* __restrict__ modal, T* __restrict__ fourier, const T* __restrict__ ptab,
     const int64_t* __restrict__ m_off, int B, int L, int J, int Jh, int Jhp, int Rrows) {
@@ -115,7 +116,6 @@ __global__ __launch_bounds__(NT) void legendre_inverse_fma_kernel(
   }
 }
 
-template <typename T>
 __global__ __launch_bounds__(NT) void legendre_forward_fma_kernel(
     const T* __restrict__ fourier, T* __restrict__ modal, const T* __restrict__ ptab,
     const int64_t* __restrict__ m_off, int B, int L, int J, int Jh, int Jhp, int Rrows) {
@@ -213,25 +213,19 @@ __global__ __launch_bounds__(NT) void legendre_forward_fma_kernel(
   }
 }
 
-template <typename T>
-int run_legendre(bool forward, const dino_plan* pl, const void* in, void* out, int64_t B,
+int run_legendre(bool forward, const dino_plan* pl, const double* in, double* out, int64_t B,
                  hipStream_t s) {
   if (B == 0) return DINO_OK;
   DINO_REQUIRE(2 * B <= (int64_t)65535 * TR, DINO_EINVAL, "batch too large");
-  const T* ptab;
-  if constexpr (sizeof(T) == 8) ptab = pl->p64;
-  else ptab = pl->p32;
   int row_tiles = (int)((2 * B + TR - 1) / TR);
   if (forward) {
     dim3 grid((pl->L + TC - 1) / TC, row_tiles, pl->M);
-    legendre_forward_fma_kernel<T><<<grid, NT, 0, s>>>(
-        static_cast<const T*>(in), static_cast<T*>(out), ptab, pl->m_offset, (int)B, pl->L,
-        pl->J, pl->Jh, pl->Jhp, pl->R);
+    legendre_forward_fma_kernel<<<grid, NT, 0, s>>>(
+        in, out, pl->p64, pl->m_offset, (int)B, pl->L, pl->J, pl->Jh, pl->Jhp, pl->R);
   } else {
     dim3 grid((pl->Jh + TC - 1) / TC, row_tiles, pl->M);
-    legendre_inverse_fma_kernel<T><<<grid, NT, 0, s>>>(
-        static_cast<const T*>(in), static_cast<T*>(out), ptab, pl->m_offset, (int)B, pl->L,
-        pl->J, pl->Jh, pl->Jhp, pl->R);
+    legendre_inverse_fma_kernel<<<grid, NT, 0, s>>>(
+        in, out, pl->p64, pl->m_offset, (int)B, pl->L, pl->J, pl->Jh, pl->Jhp, pl->R);
   }
   DINO_LAUNCH_CHECK("legendre fma kernel");
   return DINO_OK;
@@ -239,16 +233,14 @@ int run_legendre(bool forward, const dino_plan* pl, const void* in, void* out, i
 
 }  // namespace
 
-int legendre_inverse_fma(const dino_plan* pl, const void* modal, void* fourier, int64_t B,
-                         int dtype, hipStream_t s) {
-  if (dtype == DINO_F64) return run_legendre<double>(false, pl, modal, fourier, B, s);
-  return run_legendre<float>(false, pl, modal, fourier, B, s);
+int legendre_inverse_fma(const dino_plan* pl, const double* modal, double* fourier, int64_t B,
+                         hipStream_t s) {
+  return run_legendre(false, pl, modal, fourier, B, s);
 }
 
-int legendre_forward_fma(const dino_plan* pl, const void* fourier, void* modal, int64_t B,
-                         int dtype, hipStream_t s) {
-  if (dtype == DINO_F64) return run_legendre<double>(true, pl, fourier, modal, B, s);
-  return run_legendre<float>(true, pl, fourier, modal, B, s);
+int legendre_forward_fma(const dino_plan* pl, const double* fourier, double* modal, int64_t B,
+                         hipStream_t s) {
+  return run_legendre(true, pl, fourier, modal, B, s);
 }
 
 }  // namespace dino

@@ -416,7 +416,7 @@ __global__ __launch_bounds__(64 * NW, (fwd_waves_per_simd<NW, KS>())) void leg_f
 // per workgroup: the table of a large grid (262 MB at TL639) is the largest
 // operand at common batches, so a workgroup takes as many rows of one m as
 // there are, up to 128.  2 ks of the KT node groups are in use, a half in each chain.
-// TL639, 37 fields: 519 us with the tiled kernel, 223 us here (table and rows
+// TL639, 37 fields: 519 us with the tiled kernel, 214 us here (table and rows
 // 0.08 ms at the copy rate, 10.6 GFLOP of tiles 0.07 ms).
 template <int KT, int NS, bool VIN>
 __global__ __launch_bounds__(128 * NS) void leg_fwd_split_rows_kernel(

@@ -14,8 +14,8 @@ static __device__ __align__(256) unsigned char scratch[DINO_SHT_SCRATCH_BYTES];
 namespace dino {
 int dft_forward_impl(const dino_plan*, const void*, void*, int64_t, int, int, hipStream_t);
 int dft_inverse_impl(const dino_plan*, const void*, void*, int64_t, int, int, hipStream_t);
-int legendre_inverse_fma(const dino_plan*, const void*, void*, int64_t, int, hipStream_t);
-int legendre_forward_fma(const dino_plan*, const void*, void*, int64_t, int, hipStream_t);
+int legendre_inverse_fma(const dino_plan*, const double*, double*, int64_t, hipStream_t);
+int legendre_forward_fma(const dino_plan*, const double*, double*, int64_t, hipStream_t);
 bool legendre_f64_forward_pays(const dino_plan*, int64_t);
 bool legendre_f64_inverse_pays(const dino_plan*, int64_t);
 int legendre_inverse_f64(const dino_plan*, const double*, double*, int64_t, hipStream_t);
@@ -47,7 +47,8 @@ int leg_inverse(const dino_plan* p, const void* in, void* out, int64_t B, int dt
                 hipStream_t s) {
   if (dtype == DINO_F64 && legendre_f64_inverse_pays(p, B))
     return legendre_inverse_f64(p, static_cast<const double*>(in), static_cast<double*>(out), B, s);
-  if (dtype == DINO_F64) return legendre_inverse_fma(p, in, out, B, dtype, s);
+  if (dtype == DINO_F64)
+    return legendre_inverse_fma(p, static_cast<const double*>(in), static_cast<double*>(out), B, s);
   return legendre_inverse_mfma(p, in, out, B, prec, s);
 }
 
@@ -58,7 +59,8 @@ int leg_forward(const dino_plan* p, const void* in, void* out, int64_t B, int dt
   if (dtype == DINO_F64 && legendre_f64_forward_pays(p, B))
     return legendre_forward_f64(p, static_cast<const double*>(in), static_cast<double*>(out), B,
                                 triangle_only, s);
-  if (dtype == DINO_F64) return legendre_forward_fma(p, in, out, B, dtype, s);
+  if (dtype == DINO_F64)
+    return legendre_forward_fma(p, static_cast<const double*>(in), static_cast<double*>(out), B, s);
   return legendre_forward_mfma(p, in, out, B, prec, triangle_only, s);
 }
 
