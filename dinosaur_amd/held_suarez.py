@@ -126,7 +126,9 @@ class HeldSuarezForcingSigma(time_integration.ExplicitODE):
     own = (isinstance(equation, pe) and type(self) is HeldSuarezForcingSigma
            and eq.explicit_terms is pe.explicit_terms
            and eq._explicit_fused is pe._explicit_fused
-           and not {'explicit_terms', 'equilibrium_temperature'} & set(self.__dict__))
+           and not {'explicit_terms', 'equilibrium_temperature', 'kv', 'kt'} & set(self.__dict__)
+           and not {'explicit_terms', '_explicit_fused', 'implicit_terms',
+                    'implicit_inverse'} & set(equation.__dict__))
     if not own or not equation.fused_nodal:
       return None
     a, b = self.coords, equation.coords

@@ -102,6 +102,8 @@ def compose_equations(equations: Sequence[Any]) -> ImplicitExplicitODE:
     def flat_imex_ops(state):
       fused = fuse(main)
       return None if fused is None else fused.flat_imex_ops(state)
+    # it stands for these methods only (imex_runge_kutta)
+    flat_imex_ops.methods = (out.explicit_terms, out.implicit_terms, out.implicit_inverse)
     out._flat_imex_ops = flat_imex_ops
   return out
 
@@ -541,6 +543,8 @@ def imex_runge_kutta(tableau: ImExButcherTableau, equation, time_step: float):
   n = len(b_ex)
 
   hook = getattr(equation, '_flat_imex_ops', None)
+  if getattr(hook, 'methods', (F, G, G_inv)) != (F, G, G_inv):
+    hook = None  # a method of a composed equation was replaced
 
   def fused(y0, filter_fn):
     """(flat y0, fused step output or None)."""

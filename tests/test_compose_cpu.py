@@ -1,0 +1,59 @@
+"""compose_equations of the primitive equations and the Held-Suarez forcing:
+the fused step serves only the two classes' own methods (host side)."""
+import copy
+
+import numpy as np
+import pytest
+
+from dinosaur_amd import coordinate_systems, held_suarez, primitive_equations as pe
+from dinosaur_amd import sigma_coordinates, spherical_harmonic as sh, time_integration as ti, units
+
+
+def _pair(K=4):
+  coords = coordinate_systems.CoordinateSystem(
+      sh.Grid(8, 9, 24, 12), sigma_coordinates.SigmaCoordinates.equidistant(K))
+  ps = units.SimUnits.from_si()
+  tref = np.full(K, 288.0)
+  eq = pe.PrimitiveEquationsSigma(tref, np.zeros(coords.horizontal.modal_shape), coords, ps)
+  return eq, held_suarez.HeldSuarezForcingSigma(coords, ps, tref)
+
+
+@pytest.mark.parametrize('name', ['explicit_terms', '_explicit_fused', 'implicit_terms',
+                                  'implicit_inverse'])
+def test_methods_replaced_on_the_equation_stay_unfused(name):
+  eq, hs = _pair()
+  assert hs.fused_with(eq) is not None
+  setattr(eq, name, getattr(eq, name))
+  assert hs.fused_with(eq) is None
+
+
+@pytest.mark.parametrize('name', ['explicit_terms', 'equilibrium_temperature', 'kv', 'kt'])
+def test_methods_replaced_on_the_forcing_stay_unfused(name):
+  eq, hs = _pair()
+  setattr(hs, name, getattr(hs, name))
+  assert hs.fused_with(eq) is None
+
+
+@pytest.mark.parametrize('name', ['explicit_terms', 'implicit_terms', 'implicit_inverse'])
+def test_methods_replaced_on_the_composed_equation_are_used(name, monkeypatch):
+  class Flat:
+    def as_flat(self):
+      return self
+
+  def replaced(*args):
+    raise NotImplementedError
+
+  monkeypatch.setattr(held_suarez._ForcedEquations, 'flat_imex_ops', lambda self, state: 'ops')
+  monkeypatch.setattr(ti, '_fused_imex_step', lambda *args: 'fused')
+  eq, hs = _pair()
+  monkeypatch.setattr(pe.PrimitiveEquationsSigma, 'implicit_inverse', lambda *args: 0.0)
+  composed = ti.compose_equations([eq, hs])
+  assert ti.imex_rk_sil3(composed, 0.1)(Flat()) == 'fused'
+  mine = copy.copy(composed)
+  setattr(mine, name, replaced)
+  for other in {'explicit_terms', 'implicit_terms'} - {name}:
+    setattr(mine, other, lambda state: 0.0)
+  monkeypatch.setattr(ti, '_stage', lambda *args: 0.0)
+  with pytest.raises(NotImplementedError):
+    ti.imex_rk_sil3(mine, 0.1)(Flat())
+  assert ti.imex_rk_sil3(composed, 0.1)(Flat()) == 'fused'
