@@ -1145,7 +1145,7 @@ class PrimitiveEquationsSigma:
     sh = self.coords.horizontal.spherical_harmonics
     if (type(sh) is not spherical_harmonic.RealSphericalHarmonics or not _plain(buf)
         or type(self)._explicit_fused is not PrimitiveEquationsSigma._explicit_fused
-        or not buf.is_contiguous() or buf.dtype not in (torch.float32, torch.float64)):
+        or '_explicit_fused' in self.__dict__ or not buf.is_contiguous() or buf.dtype not in (torch.float32, torch.float64)):
       return None
     plan = sh.plan(buf.device)
     if plan.tuned:

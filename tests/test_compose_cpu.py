@@ -4,6 +4,7 @@ import copy
 
 import numpy as np
 import pytest
+import torch
 
 from dinosaur_amd import coordinate_systems, held_suarez, primitive_equations as pe
 from dinosaur_amd import sigma_coordinates, spherical_harmonic as sh, time_integration as ti, units
@@ -57,3 +58,9 @@ def test_methods_replaced_on_the_composed_equation_are_used(name, monkeypatch):
   with pytest.raises(NotImplementedError):
     ti.imex_rk_sil3(mine, 0.1)(Flat())
   assert ti.imex_rk_sil3(composed, 0.1)(Flat()) == 'fused'
+
+
+def test_explicit_fused_replaced_on_the_equation_is_not_one_call():
+  eq, _ = _pair()
+  eq._explicit_fused = lambda *args: None
+  assert eq._native_args(torch.zeros(13, 15, 9), 1, []) is None
