@@ -86,12 +86,14 @@ __global__ __launch_bounds__(256) void leg_fwd_f64_kernel(
     row_field(m, row, &b, &r);
     return modal + ((int64_t)b * Rrows + r) * L;
   };
-  if (blockIdx.z == 0 && !skip_zero) {
+  // zeros below the triangle; with skip_zero only from the first tile's degree on
+  if (blockIdx.z == 0) {
+    const int l0 = skip_zero ? leg_tile_start(m, L) : 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       double* const o = out_row(i);
       if (o)
-        for (int l = 2 * c16 + par; l < m; l += 32) o[l] = 0.0;
+        for (int l = l0 + 2 * c16 + par; l < m; l += 32) o[l] = 0.0;
     }
   }
   const double* const pm = p64 + m_off[m];

@@ -53,7 +53,7 @@ int leg_inverse(const dino_plan* p, const void* in, void* out, int64_t B, int dt
 }
 
 // triangle_only: rows may skip the all-zero degrees below leg_tile_start(m, L)
-// (the FP64 and tiled kernels write them anyway, which is also allowed).
+// (the tiled and FMA kernels write them anyway, which is also allowed).
 int leg_forward(const dino_plan* p, const void* in, void* out, int64_t B, int dtype, int prec,
                 hipStream_t s, bool triangle_only = false) {
   if (dtype == DINO_F64 && legendre_f64_forward_pays(p, B))

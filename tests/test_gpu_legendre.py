@@ -94,3 +94,30 @@ def test_legendre_matches_table(gpu_device, nodes, odd):
           assert (buf[:skew] == 7.0).all() and (buf[skew + dst.size:] == 7.0).all()
   for stage in (_lib.STAGE_LEGENDRE_INVERSE, _lib.STAGE_LEGENDRE_FORWARD):
     plan.set_schedule(stage, 0)
+
+
+# Northern nodes of each forward kernel: row-resident, split, tiled; FP64 on the
+# matrix cores (4, 8, 16 node groups) and in FMA tiles (257 up).
+@pytest.mark.parametrize('nodes', [16, 65, 129, 256, 257, 513])
+@pytest.mark.parametrize('code,prec', [(_lib.DINO_F32, _lib.PREC_NATIVE),
+                                       (_lib.DINO_F32, _lib.PREC_BF16X3),
+                                       (_lib.DINO_F64, _lib.PREC_NATIVE)])
+def test_triangle_only_rows_are_whole_from_their_first_tile(gpu_device, nodes, code, prec):
+  M, L, J = 40, 75, 2 * nodes
+  print('[test] triangle only', nodes, code, prec, flush=True)
+  plan = sh.get_plan(M, L, 2 * M, J, 'gauss', gpu_device)
+  dtype = torch.float32 if code == _lib.DINO_F32 else torch.float64
+  lib, p = _lib.lib(), lambda t: ctypes.c_void_p(t.data_ptr())
+  stream = ctypes.c_void_p(torch.cuda.current_stream(gpu_device).cuda_stream)
+  m = (torch.arange(plan.R, device=gpu_device)[:, None] + 1) // 2
+  start = (L - 32 * ((L - m + 31) // 32)).clamp(min=0)
+  l = torch.arange(L, device=gpu_device)
+  for B in (1, 40):
+    x = torch.randn((B, plan.R, J), dtype=dtype, device=gpu_device)
+    whole, part = (torch.full((B, plan.R, L), float('nan'), dtype=dtype, device=gpu_device)
+                   for _ in range(2))
+    for out, flag in ((whole, 0), (part, _lib.SHT_TRIANGLE_ONLY)):
+      _lib.check(lib.dino_legendre_forward(plan.handle, p(x), p(out), B, code, prec | flag,
+                                           stream))
+    assert (whole[:, l < m] == 0).all()
+    assert part[:, l >= start].equal(whole[:, l >= start])
