@@ -44,8 +44,14 @@ class HeldSuarezForcingSigma(time_integration.ExplicitODE):
     return self.ka + (self.ks - self.ka) * (cutoff[:, np.newaxis, np.newaxis]
                                            * np.cos(self.lat) ** 4)
 
+  def _parameters(self):
+    """What the constants below are made of, as a cache key."""
+    arrays = (self.sigma, self.reference_temperature, self.lat[0])
+    return (float(self.sigma_b), float(self.kf), float(self.ka), float(self.ks),
+            *(np.asarray(a, np.float64).tobytes() for a in arrays))
+
   def _c(self, name, like):
-    key = (name, like.device, like.dtype)
+    key = (name, like.device, like.dtype, self._parameters())
     t = self._consts.get(key)
     if t is None:
       grid = self.coords.horizontal
@@ -97,7 +103,7 @@ class HeldSuarezForcingSigma(time_integration.ExplicitODE):
     """The forcing's constants on a device, for the nodal kernels."""
     scalars = [float(x) for x in (self.minT, self.maxT, self.dTy, self.dThz,
                                   self.physics_specs.kappa, self.p0)]
-    key = (torch.device(device).index, *scalars)
+    key = (torch.device(device).index, *scalars, self._parameters())
     cache = self.__dict__.setdefault('_handles', {})
     h = cache.get(key)
     if h is None:

@@ -100,3 +100,19 @@ def test_pairs_the_kernels_do_not_serve_stay_unfused(gpu_device):
   eq.fused_nodal = True
   mine = Mine(eq.reference_temperature, eq.orography, eq.coords, eq.physics_specs)
   assert hs.fused_with(mine) is None
+
+
+@pytest.mark.parametrize('name', ['kf', 'ka', 'ks', 'sigma_b', 'sigma', 'reference_temperature',
+                                  'lat', 'minT', 'p0'])
+def test_changed_parameters_are_used(gpu_device, name):
+  """After a parameter changes, a forcing that has run equals a new one, fused
+  and by itself."""
+  eq, hs, st, coords, ps = _setup(6, 1, False, torch.float64, gpu_device)
+  run = lambda forcing: (forcing.fused_with(eq).explicit_terms(st), forcing.explicit_terms(st))  # noqa: E731
+  before = run(hs)
+  new = held_suarez.HeldSuarezForcingSigma(coords, ps, eq.reference_temperature)
+  for forcing in (hs, new):
+    setattr(forcing, name, getattr(forcing, name) * 0.9)
+  for b, x, y in zip(before, run(hs), run(new)):
+    assert all(p.equal(q) for p, q in zip(_leaves(x), _leaves(y)))
+    assert not all(p.equal(q) for p, q in zip(_leaves(b), _leaves(x)))
