@@ -73,10 +73,23 @@ __host__ __device__ inline COff coff(int K, int J) {
 constexpr int MAXTR = 6;
 
 // Waves that share a column's levels in the split forward kernel, two levels each at
-// least, and the batches it takes (measured at the kernel).
+// least.
 constexpr int kNodalWaves = 8;
+constexpr size_t kLdsBytes = 160 * 1024;  // of a CU
 inline int nodal_waves(int K) { return K / 2 < 1 ? 1 : K / 2 < kNodalWaves ? K / 2 : kNodalWaves; }
-inline bool nodal_split(int64_t columns) { return columns <= 98304; }
+// Bytes of LDS of a split block: what the column sums take of each level.
+inline size_t split_lds(int K, bool moist, size_t es) { return 64 * es * (moist ? 4 : 3) * (size_t)K; }
+// Batches the split form takes (members x columns): those of few bytes a field, the more
+// the more levels there are to share.  Whole columns / split, us: FP32 T42 L24 dry, 1
+// member (8192 columns) 29.9 / 10.8, 12 members (98304) 43.6 / 34.2, 32 (262144) 66 / 92;
+// L24 moist 98304 87 / 75, 131072 106 / 124; L12 dry 65536 19.2 / 16.9, 98304 23.0 / 25.6;
+// L5 moist 32768 14.3 / 14.1, 65536 16.4 / 17.8; L2 8192 5.3 / 5.9.  FP64 L24 dry 8192
+// 35 / 12.8, 49152 44.7 / 36.6, 65536 46.3 / 46.4, 98304 51 / 66; L12 32768 21.7 / 17.8, 49152
+// 23.5 / 25.2.  Beyond 160 KiB of LDS (FP32 above 160 moist levels): whole columns.
+inline bool nodal_split(int64_t columns, int K, bool moist, size_t es) {
+  return K >= 4 && columns * (int64_t)es <= (int64_t)24576 * (K < 16 ? K : 16) &&
+         split_lds(K, moist, es) <= kLdsBytes;
+}
 
 struct Groups {
   // input group offsets (in fields of I*J) for member stride computation
@@ -138,16 +151,29 @@ struct Params {
   double R, kappa, gcr, hcr, rvr, gcr1;
 };
 
+// Sums of the forward kernel whose rounding must not be left to the compiler, which
+// fuses products into sums as each form's code suggests: its two forms are to agree
+// bitwise.
+template <typename T>
+__device__ __forceinline__ T wind_sum(T a, T b, T c, T d) {  // a b + c d
+  return fma(a, b, c * d);
+}
+template <typename T>
+__device__ __forceinline__ T rounded_sum(T a, T b) {
+#pragma clang fp contract(off)
+  return a + b;
+}
+
 // ---------------------------------------------------------------- forward
 // Pass A forms the column totals, pass B streams the levels with a (k, k + 1)
 // window.  A thread walks all levels of its column, or (SPLIT) a block owns 64
-// columns and each of its waves a contiguous share of the levels: a wave's
-// sums meet the others' in LDS, its prefix sums start from those of the waves
-// above and the flux through its top interface is formed from the level above.
-// Whole columns stream every field once, in order, at the copy rate, but a grid
-// of a few thousand columns is then a few dozen waves in a long chain: T42
-// L24, one member (8192 columns), 31 us whole and 17 split; T85 L24 moist, 2
-// members (65536), 71 and 48; TL255 L37 moist, one member (131072), 170 and 192.
+// columns and each of its waves a contiguous share of the levels: what the sums
+// take of each level meets in LDS, every wave sums it in level order (totals, and
+// prefixes up to its first level) and forms the flux through its top interface from
+// the level above.  Both forms add the same terms in the same order, so a member's
+// values do not depend on the batch.  Whole columns stream every field once, in order,
+// at the copy rate, but a grid of a few thousand columns is then a few dozen waves in a
+// long chain (nodal_split: both sides measured).
 template <typename T, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_kernel(
     const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ cst, Groups g,
@@ -179,43 +205,50 @@ __global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_
   const T R = (T)p.R, kappa = (T)p.kappa;
   const bool moist = p.moist != 0;
   const T lp = moist ? *I_(g.lp, 1, 0) : (T)0;
-  // ---- pass A: sums of this thread's levels
+  // ---- pass A: column totals, summed in level order
   T TE = 0, TF = 0, GT = 0;
-  auto sum_level = [&](int k) {
-    T u = *I_(g.u, K, k), v = *I_(g.v, K, k), d = *I_(g.d, K, k);
-    T A = (u * gx + v * gy) * s;
-    T ds = cst[o.dsig + k];
-    TE += A * ds;
-    TF += (d + A) * ds;
-    if (moist && k >= 1) {
-      T q = *I_(g.tr[p.hum], K, k), t = *I_(g.t, K, k);
-      T td = q * (t + cst[o.tref + k]) * (T)p.gcr1;
-      GT += cst[o.gp + k] * td;
-    }
+  T PE = 0, PF = 0, GP = 0;  // prefixes at k; GP: sum_{1 <= h <= k} gp[h] td[h]
+  // adds level k to a pair of sums of v . grad ln ps (w: before the factor sec^2) and
+  // of that + div
+  auto add_level = [&](int k, T w, T d, T* e, T* f) {
+    const T ds = cst[o.dsig + k];
+    *e = fma(w * s, ds, *e);
+    *f = fma(fma(w, s, d), ds, *f);
+  };
+  auto moist_term = [&](int k) {
+    const T q = *I_(g.tr[p.hum], K, k), t = *I_(g.t, K, k);
+    return q * (t + cst[o.tref + k]) * (T)p.gcr1;
   };
   if constexpr (SPLIT) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    // what the sums take of each level: w of the totals, w of the prefixes (they
+    // round differently, see wind_sum), d, td
+    T* const lev = reinterpret_cast<T*>(smem_raw) + lane;
+    const int P = 64 * K;
 #pragma unroll 4
-    for (int k = k0; k < k1; ++k) sum_level(k);
-  } else {
-    for (int k = 0; k < K; ++k) sum_level(k);
-  }
-  T PE = 0, PF = 0, GP = 0;  // prefixes at k; GP: sum_{1 <= h <= k} gp[h] td[h]
-  if constexpr (SPLIT) {
-    __shared__ T part[3][kNodalWaves][64];
-    part[0][wave][lane] = TE;
-    part[1][wave][lane] = TF;
-    part[2][wave][lane] = GT;
+    for (int k = k0; k < k1; ++k) {
+      const T u = *I_(g.u, K, k), v = *I_(g.v, K, k);
+      lev[64 * k] = wind_sum(u, gx, v, gy);
+      lev[64 * k + P] = wind_sum(v, gy, u, gx);
+      lev[64 * k + 2 * P] = *I_(g.d, K, k);
+      if (moist) lev[64 * k + 3 * P] = moist_term(k);
+    }
     __syncthreads();
-    TE = TF = GT = 0;
-    for (int i = 0; i < G; ++i) {
-      if (i == wave) {
-        PE = TE;
-        PF = TF;
-        GP = GT;
+    // the totals, and the prefixes up to this wave's first level
+    for (int k = 0; k < K; ++k) {
+      const T d = lev[64 * k + 2 * P];
+      add_level(k, lev[64 * k], d, &TE, &TF);
+      if (k < k0) add_level(k, lev[64 * k + P], d, &PE, &PF);
+      if (moist) {
+        if (k == k0) GP = GT;
+        if (k >= 1) GT = fma(cst[o.gp + k], lev[64 * k + 3 * P], GT);
       }
-      TE += part[0][i][lane];
-      TF += part[1][i][lane];
-      GT += part[2][i][lane];
+    }
+  } else {
+    for (int k = 0; k < K; ++k) {
+      const T u = *I_(g.u, K, k), v = *I_(g.v, K, k);
+      add_level(k, wind_sum(u, gx, v, gy), *I_(g.d, K, k), &TE, &TF);
+      if (moist && k >= 1) GT = fma(cst[o.gp + k], moist_term(k), GT);
     }
   }
   if (wave == 0) put(g.lsp, 1, 0, -TE);
@@ -258,9 +291,9 @@ __global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_
     }
     const T d = *I_(g.d, K, k), z = *I_(g.z, K, k);
     const T ds = cst[o.dsig + k];
-    const T A = (u0 * gx + v0 * gy) * s;
-    PE += A * ds;
-    PF += (d + A) * ds;
+    const T w = wind_sum(v0, gy, u0, gx);
+    const T A = w * s;
+    add_level(k, w, d, &PE, &PF);
     T W = 0, X = 0;
     if (!last) {
       W = cst[o.ss + k] * TF - PF;
@@ -269,14 +302,15 @@ __global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_
     const T c = last ? (T)0 : cst[o.c2c + k];
     // vertical advection -(w dx/dsigma), averaged over the two interfaces
     T fu = W * (u1 - u0) * c, fv = W * (v1 - v0) * c, ft = W * (t1 - t0) * c;
-    T vadv_u = (T)-0.5 * (fu + fu_m), vadv_v = (T)-0.5 * (fv + fv_m);
-    T vadv_t = (T)-0.5 * (ft + ft_m);
+    T vadv_u = (T)-0.5 * fma(W * (u1 - u0), c, fu_m);
+    T vadv_v = (T)-0.5 * fma(W * (v1 - v0), c, fv_m);
+    T vadv_t = (T)-0.5 * fma(W * (t1 - t0), c, ft_m);
     T tref = cst[o.tref + k];
     T vadv_x = 0;
     if (p.tnc) {
       T tref1 = last ? (T)0 : cst[o.tref + k + 1];
       T fx = last ? (T)0 : X * (tref1 - tref) * c;
-      vadv_x = (T)-0.5 * (fx + fx_m);
+      vadv_x = (T)-0.5 * rounded_sum(fx, fx_m);
       fx_m = fx;
     }
     // humidity
@@ -316,7 +350,7 @@ __global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_
       if (i < p.nt) {
         T x0 = tr0[i];
         T fx = W * (tr1[i] - x0) * c;
-        T va = (T)-0.5 * (fx + ftr_m[i]);
+        T va = (T)-0.5 * fma(W * (tr1[i] - x0), c, ftr_m[i]);
         ftr_m[i] = fx;
         put(g.trn[i], K, k, (iva ? va : (T)0) + x0 * d);
         put(g.tu[i], K, k, u0 * x0 * s);
@@ -327,9 +361,9 @@ __global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_
       T qx = *I_(g.qx, K, k), qy = *I_(g.qy, K, k);
       T cf = tref * (T)p.rvr;
       put(g.curl, K, k, cf * s * (gx * qy - gy * qx));
-      put(g.dc, K, k, cf * s * (qx * gx + qy * gy) + q * lp * tref * (T)p.rvr);
+      put(g.dc, K, k, fma(q * lp * tref, (T)p.rvr, cf * s * wind_sum(qx, gx, qy, gy)));
       T td = q * (t0 + tref) * (T)p.gcr1;
-      if (k >= 1) GP += cst[o.gp + k] * td;
+      if (k >= 1) GP = fma(cst[o.gp + k], td, GP);
       put(g.ke, K, k, kinetic + (cst[o.gd + k] * td + (GT - GP)));
     }
     fu_m = fu;
@@ -698,11 +732,15 @@ int launch(bool adjoint, const dino_nodal* n, const void* in, const void* gout, 
   if constexpr (sizeof(T) == 8) cst = n->c64;
   else cst = n->c32;
   dim3 grid((unsigned)((p.IJ + 255) / 256), (unsigned)E);
-  if (!adjoint && nodal_split(p.IJ * E))
+  const size_t lds = split_lds(p.K, p.moist != 0, sizeof(T));
+  if (!adjoint && nodal_split(p.IJ * E, p.K, p.moist != 0, sizeof(T))) {
+    if (lds > 65536)
+      DINO_HIP(hipFuncSetAttribute((const void*)nodal_forward_kernel<T, true>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     nodal_forward_kernel<T, true><<<dim3((unsigned)((p.IJ + 63) / 64), (unsigned)E),
-                                    dim3(64, (unsigned)nodal_waves(p.K)), 0, s>>>(
+                                    dim3(64, (unsigned)nodal_waves(p.K)), lds, s>>>(
         static_cast<const T*>(in), static_cast<T*>(out), cst, g, p);
-  else if (!adjoint)
+  } else if (!adjoint)
     nodal_forward_kernel<T, false><<<grid, 256, 0, s>>>(static_cast<const T*>(in),
                                                         static_cast<T*>(out), cst, g, p);
   else

@@ -73,6 +73,23 @@ def test_member_in_group_matches_member_alone(gpu_device):
       assert ((x - y).abs().max() / scale).item() <= 1e-6, k
 
 
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
+def test_member_equals_member_alone_across_kernel_choices(gpu_device, dtype):
+  """16 members of T42 L12 take other nodal, implicit and modal launch shapes than
+  one; a step of a member is bitwise the same in both."""
+  eq, st, coords, ps = workloads.build_primitive('T42', 12, moist=True, members=16, dtype=dtype,
+                                                 device=gpu_device)
+  dt = ps.nondimensionalize(600.0 * units_lib.scales.units.s)
+  step = ti.step_with_filters(ti.imex_rk_sil3(eq, dt),
+                              [ti.exponential_step_filter(coords.horizontal, dt)])
+  whole, alone = step(step(st)), st.tree_map_arrays(lambda x: x[7:8])
+  alone = step(step(alone))
+  for f in alone._ARRAYS:
+    assert getattr(whole, f)[7:8].equal(getattr(alone, f)), f
+  for k, x in alone.tracers.items():
+    assert whole.tracers[k][7:8].equal(x), k
+
+
 def test_config3_mixed_ensemble_graph_ticks(gpu_device):
   """The 64-member mixed ensemble (32 T85 + 24 T42 + 8 TL127, moist L24, 10 min
   steps, T42 at 20 min every other tick): 4 graphed ticks on concurrent
