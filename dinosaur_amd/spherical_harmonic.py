@@ -1050,7 +1050,8 @@ def _winds_handle(grid: Grid, a: torch.Tensor, b: torch.Tensor, tail):
   sh = grid.spherical_harmonics
   if (type(sh) is not RealSphericalHarmonics or a.shape != b.shape or a.dtype != b.dtype
       or a.device != b.device or a.dtype not in (torch.float32, torch.float64)
-      or tuple(a.shape[-2:]) != tuple(tail) or a.numel() == 0):
+      or tuple(a.shape[-2:]) != tuple(tail) or a.numel() == 0
+      or sh.total_wavenumbers < 2):  # the operators' kernels need two degrees
     return None
   key = (grid, 'winds', a.device)
   h = _const_cache.get(key)

@@ -92,3 +92,14 @@ def test_winds_outputs_are_independent(gpu_device):
   torch.autograd.grad(w + u.sum(), x)
   out = sh.vor_div_to_uv_nodal(grid, z.cpu().numpy(), z.cpu().numpy())
   assert all(isinstance(a, np.ndarray) for a in out)
+
+
+def test_one_degree_takes_the_composed_operators(gpu_device):
+  grid = sh.Grid(1, 1, 4, 2)
+  z, d = (torch.randn((3, 1, 1), device=gpu_device) for _ in range(2))
+  for a, b in zip(sh.vor_div_to_uv_nodal(grid, z, d), _composed_uv(grid, z, d, True)):
+    assert a.shape == (3, 4, 2) and a.equal(b)
+  u, v = (torch.randn((3, 4, 2), device=gpu_device) for _ in range(2))
+  for a, b in zip(sh.uv_nodal_to_vor_div_modal(grid, u, v, clip=False),
+                  _composed_vor_div(grid, u, v, False)):
+    assert a.shape == (3, 1, 1) and a.equal(b)
