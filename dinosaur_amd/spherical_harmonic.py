@@ -1037,11 +1037,13 @@ class _Winds(torch.autograd.Function):
 
 
 def _pair_of(x, lead, tail):
-  """The two fields of a (2B, ...) buffer; tensors of their own when autograd
-  follows them, so that one may be changed in place without the other."""
+  """The two fields of a (2B, ...) buffer as tensors that can be changed in place
+  one without the other: with memory of their own when autograd follows them, else
+  halves of the buffer with a version counter each (`data`; views would share one,
+  and autograd would refuse a product of u after a change of v)."""
   a, b = (x[i * (x.shape[0] // 2):(i + 1) * (x.shape[0] // 2)].reshape(lead + tail)
           for i in (0, 1))
-  return (a.clone(), b.clone()) if x.requires_grad else (a, b)
+  return (a.clone(), b.clone()) if x.requires_grad else (a.data, b.data)
 
 
 def _winds_handle(grid: Grid, a: torch.Tensor, b: torch.Tensor, tail):

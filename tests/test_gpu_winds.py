@@ -103,3 +103,15 @@ def test_one_degree_takes_the_composed_operators(gpu_device):
   for a, b in zip(sh.uv_nodal_to_vor_div_modal(grid, u, v, clip=False),
                   _composed_vor_div(grid, u, v, False)):
     assert a.shape == (3, 1, 1) and a.equal(b)
+
+
+def test_changing_one_output_leaves_the_other_usable_by_autograd(gpu_device):
+  grid = GRIDS[0]
+  z = torch.randn((2,) + grid.modal_shape, device=gpu_device)
+  w = torch.randn((2,) + grid.nodal_shape, device=gpu_device)
+  for a, b in (sh.vor_div_to_uv_nodal(grid, z, z), sh.uv_nodal_to_vor_div_modal(grid, w, w)):
+    a.requires_grad_()
+    y = (a * a).sum()
+    b.mul_(2.0)
+    y.backward()
+    assert a.grad.equal(2 * a.detach())
