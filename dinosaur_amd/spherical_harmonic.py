@@ -1046,6 +1046,13 @@ def _pair_of(x, lead, tail):
   return (a.clone(), b.clone()) if x.requires_grad else (a.data, b.data)
 
 
+# Handles of the wind kernels, kept like the plans (captured graphs read their
+# constants) and under what those are made of: grids that compare unequal only by
+# their implementation object share one (59 MB at TL639).
+_winds_handles: dict = {}
+_winds_lock = threading.Lock()
+
+
 def _winds_handle(grid: Grid, a: torch.Tensor, b: torch.Tensor, tail):
   """The grid's operator handle when the fused wind kernels serve this pair of
   tensors (Real layout, one shape, float type and device), else None."""
@@ -1055,12 +1062,12 @@ def _winds_handle(grid: Grid, a: torch.Tensor, b: torch.Tensor, tail):
       or tuple(a.shape[-2:]) != tuple(tail) or a.numel() == 0
       or sh.total_wavenumbers < 2):  # the operators' kernels need two degrees
     return None
-  key = (grid, 'winds', a.device)
-  h = _const_cache.get(key)
-  if h is None:
-    from .primitive_equations import modal_handle  # pylint: disable=import-outside-toplevel
-    h = modal_handle(grid, 1, 0, -1, 0.0, a.device)
-    _const_cache[key] = h
+  key = (sh.modal_shape, float(grid.radius), a.device)
+  with _winds_lock:
+    h = _winds_handles.get(key)
+    if h is None:
+      from .primitive_equations import modal_handle  # pylint: disable=import-outside-toplevel
+      h = _winds_handles[key] = modal_handle(grid, 1, 0, -1, 0.0, a.device)
   return h
 
 

@@ -7,6 +7,8 @@ Tolerance, normwise: 1e-12 in FP64 (1e-9 on the equiangular grid, whose
 quadrature weights and 1 / cos(lat) span nine decades), 2e-3 in FP32 for the
 divergence, a small difference of large terms (2e-5 for the winds).
 """
+import functools
+
 import numpy as np
 import pytest
 import torch
@@ -115,3 +117,15 @@ def test_changing_one_output_leaves_the_other_usable_by_autograd(gpu_device):
     b.mul_(2.0)
     y.backward()
     assert a.grad.equal(2 * a.detach())
+
+
+def test_equal_grids_share_one_handle(gpu_device):
+  """Also grids made with a functools.partial of their own, which compare unequal."""
+  def handle(**kw):
+    impl = functools.partial(sh.RealSphericalHarmonics, transform_precision='float32')
+    grid = sh.Grid(8, 9, 24, 12, spherical_harmonics_impl=impl, **kw)
+    z = torch.zeros((1,) + grid.modal_shape, device=gpu_device)
+    return sh._winds_handle(grid, z, z, grid.modal_shape)
+
+  first = handle()
+  assert handle() is first and handle(radius=2.0) is not first
