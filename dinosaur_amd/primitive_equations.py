@@ -1140,8 +1140,8 @@ class PrimitiveEquationsSigma:
     """Arguments of the one-call explicit terms on a flat state buffer, or None
     where they do not apply: under autograd and its transforms, with tuned
     launch schedules (set per transform and batch), or replaced methods or
-    transforms.  The tensors and handles they point to live in this object's
-    caches and the caller's buffers."""
+    transforms.  They hold the tensors and handles that they point to, but for
+    the caller's buffers."""
     sh = self.coords.horizontal.spherical_harmonics
     if (type(sh) is not spherical_harmonic.RealSphericalHarmonics or not _plain(buf)
         or type(self)._explicit_fused is not PrimitiveEquationsSigma._explicit_fused
@@ -1154,12 +1154,17 @@ class PrimitiveEquationsSigma:
     oro = self._orography_modal(buf)
     if not oro.is_contiguous():
       return None
-    return _lib.ExplicitArgs(
-        plan.handle, self._modal_handle(buf.device, names, flags).handle,
-        self._nodal_handle(buf.device, names).handle,
-        forcing.handle(buf.device).handle if forcing is not None else None, oro.data_ptr(),
+    owners = (plan, self._modal_handle(buf.device, names, flags),
+              self._nodal_handle(buf.device, names),
+              forcing.handle(buf.device) if forcing is not None else None, oro)
+    args = _lib.ExplicitArgs(
+        *(h.handle if h is not None else None for h in owners[:4]), oro.data_ptr(),
         members, self.coords.vertical.layers, len(names),
         _lib.DINO_F64 if buf.dtype == torch.float64 else _lib.DINO_F32, sh._precision)
+    # what the pointers belong to lives as long as they do, whatever another thread
+    # puts in the caches meanwhile
+    args.owners = owners
+    return args
 
   @property
   def _modal_moist(self) -> bool:

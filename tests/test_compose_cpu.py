@@ -1,6 +1,9 @@
 """compose_equations of the primitive equations and the Held-Suarez forcing:
-the fused step serves only the two classes' own methods (host side)."""
+the fused step serves only the two classes' own methods, and the arguments of
+its one-call form hold what they point to (host side)."""
 import copy
+import gc
+import weakref
 
 import numpy as np
 import pytest
@@ -64,3 +67,25 @@ def test_explicit_fused_replaced_on_the_equation_is_not_one_call():
   eq, _ = _pair()
   eq._explicit_fused = lambda *args: None
   assert eq._native_args(torch.zeros(13, 15, 9), 1, []) is None
+
+
+def test_one_call_arguments_hold_what_they_point_to(monkeypatch):
+  """A handle that another thread drops from the caches stays alive with them."""
+  class Handle:
+    handle, tuned = 1, None
+
+  eq, hs = _pair()
+  monkeypatch.setattr(sh.RealSphericalHarmonics, 'plan', lambda self, device: Handle())
+  made = []
+
+  def make(*args):
+    h = Handle()
+    made.append(weakref.ref(h))
+    return h
+
+  eq._modal_handle = eq._nodal_handle = hs.handle = make
+  args = eq._native_args(torch.zeros(13, 15, 9), 1, [], hs)
+  eq._consts.clear()
+  gc.collect()
+  assert len(made) == 3 and all(r() is not None for r in made)
+  assert any(isinstance(t, torch.Tensor) and t.data_ptr() == args.orography for t in args.owners)
