@@ -742,8 +742,7 @@ class _FlatImexOps:
     # explicit terms when they run the fused modal kernels (which read
     # l >= m only); the tensor-op path's derivative recurrences would
     # multiply those entries by zero coefficients.
-    self.stage_triangle_only = (real and eq.fused_nodal and
-                                type(eq).explicit_terms is PrimitiveEquationsSigma.explicit_terms)
+    self.stage_triangle_only = real and fused and '_explicit_fused' not in eq.__dict__
 
   def native_step(self, buf, tab, dt, scale):
     """One whole step in one call (dino_imex_step), or None where that does not
@@ -1145,7 +1144,8 @@ class PrimitiveEquationsSigma:
     sh = self.coords.horizontal.spherical_harmonics
     if (type(sh) is not spherical_harmonic.RealSphericalHarmonics or not _plain(buf)
         or type(self)._explicit_fused is not PrimitiveEquationsSigma._explicit_fused
-        or '_explicit_fused' in self.__dict__ or not buf.is_contiguous() or buf.dtype not in (torch.float32, torch.float64)):
+        or '_explicit_fused' in self.__dict__ or not buf.is_contiguous()
+        or buf.dtype not in (torch.float32, torch.float64)):
       return None
     plan = sh.plan(buf.device)
     if plan.tuned:

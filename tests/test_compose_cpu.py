@@ -89,3 +89,13 @@ def test_one_call_arguments_hold_what_they_point_to(monkeypatch):
   gc.collect()
   assert len(made) == 3 and all(r() is not None for r in made)
   assert any(isinstance(t, torch.Tensor) and t.data_ptr() == args.orography for t in args.owners)
+
+
+@pytest.mark.parametrize('name', ['explicit_terms', '_explicit_fused'])
+def test_replaced_explicit_terms_get_whole_stage_values(name):
+  """Stage values may leave the entries below the triangle unwritten only for the
+  kernels that skip them."""
+  eq, _ = _pair()
+  assert pe._FlatImexOps(eq, ((), 4, ()), 1).stage_triangle_only
+  setattr(eq, name, getattr(eq, name))
+  assert not pe._FlatImexOps(eq, ((), 4, ()), 1).stage_triangle_only
