@@ -8,9 +8,9 @@
 // (the algorithmic minimum), versus the reference's dense (I x 2M-1) matmul
 // (spherical_harmonic.py:266-268, 275-276).
 //
-// Other I: a mixed-radix FFT when every prime factor is 2, 3, 5 or 7
-// (dft_mixed.hip), else a folded real DFT on the matrix cores up to 513
-// longitudes (dft_gemm.hip).  What remains (longer lengths with a large prime
+// Other I from 64 on: a mixed-radix FFT when every prime factor is 2, 3, 5 or 7
+// (dft_mixed.hip).  Shorter I, and those of larger factors up to 513: a folded real DFT
+// on the matrix cores (dft_gemm.hip).  What remains (longer lengths with a large prime
 // factor, fewer than 8 longitudes): a direct real DFT with the cos/sin table in
 // LDS, O(I M) per column.
 //

@@ -1,6 +1,6 @@
 // Longitude transform of lengths up to 513 with a prime factor above 7 (67,
-// 268, 341, 511, ...: grids of 2M + 1 or 3M + 1 longitudes) as a folded real DFT
-// on the matrix cores.
+// 268, 341, 511, ...: grids of 2M + 1 or 3M + 1 longitudes), and of all lengths from 8
+// to 63 but powers of two, as a folded real DFT on the matrix cores.
 //
 // With e_n = x_n + x_{N-n} and o_n = x_n - x_{N-n} (0 < n < N / 2) the rows are
 //   cos row m = s_m (x_0 + (-1)^m x_{N/2}) + sum_n s_m cos(2 pi m n / N) e_n,
@@ -233,6 +233,15 @@ int gemm_by_groups(const T* in, T* out, const T* tab, const T* qw, const GemmArg
 bool dft_gemm_available(int I, int M) {
   return M >= 2 && I >= 8 && I <= 2 * 16 * kMaxGroups + 1 && M - 1 <= 16 * kMaxGroups;
 }
+
+// Lengths of factors 2, 3, 5, 7 that take this kernel rather than the mixed-radix FFT
+// (dft_mixed.hip), whose passes are a chain of barriers however short the column is.
+// Below 64 it is the faster one in both types at every batch; beyond, not for few
+// fields in FP64.  Forward, FFT / here, us: I = 30, FP32, 12 fields 15.7 / 3.8, 1000 10.1 /
+// 4.1; I = 45 13.6 / 4.7, 9.9 / 5.8, FP64 11.4 / 6.4, 10.9 / 7.9; I = 63 17.8 / 4.7, 12.6 / 6.6,
+// 19.7 / 6.7, 15.8 / 9.8; I = 72 6.7 / 6.0, 12.7 / 11.0, 8.3 / 9.8, 20.5 / 19.7.  (The direct
+// kernel: I = 30 7.5 and 11.0, I = 45 12.2 and 19.7.)
+bool dft_gemm_short(int I) { return I < 64; }
 
 int64_t dft_gemm_table_elems(const dino_plan* pl, bool inverse) {
   return (int64_t)gemm_tiles(pl, inverse) * 2 * gemm_groups(pl, inverse) * 256;

@@ -1,4 +1,4 @@
-// Longitude transform for smooth I that is no power of two (96, 192, 320,
+// Longitude transform for smooth I from 64 on that is no power of two (96, 192, 320,
 // 360, 640, 1280, ... : every factor 2, 3, 5 or 7): mixed-radix Stockham FFT
 // in LDS, same packing and unpacking as dft.hip (two real latitude columns
 // form one complex column).

@@ -160,6 +160,7 @@ __global__ void latitude_weights_kernel(int I, int J, int stride, const double* 
 
 bool dft_mixed_available(int N, bool f64);
 bool dft_gemm_available(int I, int M);
+bool dft_gemm_short(int I);
 int64_t dft_gemm_table_elems(const dino_plan* pl, bool inverse);
 void dft_gemm_table_fill(const dino_plan* pl, hipStream_t s);
 int forward_fragment_steps(int Jh);
@@ -279,7 +280,8 @@ extern "C" int dino_plan_create(int M, int L, int I, int J, const double* nodes,
   PLAN_HIP(hipGetLastError());
   twiddle_kernel<<<(I + 255) / 256, 256>>>(I, p->tw64, p->tw32);
   PLAN_HIP(hipGetLastError());
-  if (!p->pow2 && !dft_mixed_available(I, false) && dft_gemm_available(I, M)) {
+  if (!p->pow2 && (dft_gemm_short(I) || !dft_mixed_available(I, false)) &&
+      dft_gemm_available(I, M)) {
     for (int inv = 0; inv < 2; ++inv) {
       const int64_t n = dft_gemm_table_elems(p, inv);
       PLAN_HIP(hipMalloc(&p->dftg32[inv], sizeof(float) * n));

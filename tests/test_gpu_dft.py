@@ -26,6 +26,8 @@ SHAPES = [
     (2560, 1280, 9), (4096, 2048, 4), (64, 22, 32), (512, 256, 36), (1024, 341, 10),
     (2048, 1000, 6), (11, 6, 3), (67, 22, 34), (268, 89, 134), (341, 170, 171), (511, 170, 256),
     (127, 64, 64), (202, 101, 16), (583, 291, 40), (9, 1, 6),
+    # the last smooth lengths of the matrix cores and the first of the mixed-radix FFT
+    (60, 20, 30), (63, 32, 31), (70, 35, 9), (9, 5, 3), (45, 23, 23), (45, 1, 22),
 ]
 
 
