@@ -188,7 +188,9 @@ __global__ __launch_bounds__(256) void leg_inv_f64_kernel(
 template <int KT>
 int launch_fwd(const dino_plan* pl, const double* in, double* out, int64_t B, int skip,
                hipStream_t s) {
-  // four blocks a CU, splitting the degree tiles of a row block if need be
+  // up to four blocks a CU by splitting the degree tiles of a row block; its rows are
+  // then read once per part, so no more (T85, 96 fields: 21.1 us in one part, 26.7 in two,
+  // which would be 4.03 blocks a CU)
   const int64_t gx = (2 * B + 31) / 32, want = 4 * (int64_t)device_cus();
   const int tiles = (pl->L + kTile - 1) / kTile;
   const int z = (int)std::min<int64_t>(tiles, std::max<int64_t>(1, want / (gx * pl->M)));
@@ -211,24 +213,34 @@ int launch_inv(const dino_plan* pl, const double* in, double* out, int64_t B, hi
 
 }  // namespace
 
-// Row blocks over which the FMA tiles win (the comment at the top): TL255
-// forward, 222 fields, 283 us here against 413; TL639, 37 fields, 1200 against
-// 1120 (operands of 320 nodes leave one wave per SIMD).
+// By the grid alone: the two kernels add in another order, and a field's result does not
+// depend on the batch.  FMA tiles / here, us: TL255, 222 fields 413 / 283; T213 (160
+// nodes), 37 fields 143 / 66; small grids with many fields are even, T31 (24 nodes), 1000
+// fields 23.6 / 24.5, T42 35 / 33, 80 longitudes x 40 nodes 54 / 56 (500 fields 35 / 38); TL639, 37
+// fields, 1120 / 1200 (operands of 320 nodes leave one wave per SIMD).
 bool legendre_f64_forward_pays(const dino_plan* pl, int64_t B) {
   return pl->Jh <= 256 && B < (int64_t)1 << 30;
 }
 
-// T85 (64 nodes), 1000 fields, 2752 row blocks: 99 us here against 111; TL255 (128
-// nodes): 10 fields, 256 row blocks, 32 against 55, 222 fields, 1792, 248
-// against 239, 1000 fields 1085 against 995.
+// By the batch as well: both kernels add a class's products in the order of the degrees,
+// so their results are bitwise the same.  FMA tiles / here, us: T85 (64 nodes), 1000
+// fields, 2752 row blocks 98 / 87; TL255 (128 nodes), 8 fields, 256 row blocks 53 / 28, 64
+// fields, 512, 78 / 59, 300 fields, 2560, 329 / 340.  Above 128 nodes the waves of a block
+// re-read a table that the L2s do not hold (T213 29 MB, T340 119 MB), so only where a block
+// has one wave with rows (8 fields) or the row blocks are few: T213 (160 nodes), 32
+// fields, 214 row blocks 63 / 38, 37 fields, 428, 65 / 70; T340, 8 fields 79 / 59, 12 fields,
+// 341, 84 / 89; TL639, 8 fields 310 / 228, 37 fields 674 / 874.
 bool legendre_f64_inverse_pays(const dino_plan* pl, int64_t B) {
-  return B < (int64_t)1 << 30 && (pl->Jh <= 96 || (2 * B + 63) / 64 * pl->M <= 512);
+  const int64_t blocks = (2 * B + 63) / 64 * pl->M;
+  if (B >= (int64_t)1 << 30) return false;
+  return pl->Jh <= 96 || (pl->Jh <= 128 ? blocks <= 512 : B <= 8 || blocks <= 256);
 }
 
 int legendre_forward_f64(const dino_plan* pl, const double* in, double* out, int64_t B,
                          bool triangle_only, hipStream_t s) {
   if (B == 0) return DINO_OK;
   const int skip = triangle_only ? 1 : 0;
+  if (pl->Jh <= 32) return launch_fwd<2>(pl, in, out, B, skip, s);
   if (pl->Jh <= 64) return launch_fwd<4>(pl, in, out, B, skip, s);
   if (pl->Jh <= 128) return launch_fwd<8>(pl, in, out, B, skip, s);
   return launch_fwd<16>(pl, in, out, B, skip, s);
@@ -239,10 +251,11 @@ int legendre_inverse_f64(const dino_plan* pl, const double* in, double* out, int
   if (B == 0) return DINO_OK;
   // narrower node blocks re-read the modal rows but make more waves: T85, 96
   // fields (258 blocks of 64 nodes) 16.0 us with 32 nodes, 17.3 with 64; 1000
-  // fields 108 and 99
+  // fields 108 and 99.  A grid of up to 32 nodes has no use for 64: T31, 1000 fields 13.3
+  // and 19.7, T42 19.9 and 27.5
   const int64_t blocks = (2 * B + 63) / 64 * pl->M * ((pl->Jh + 63) / 64);
   if (pl->Jh <= 16) return launch_inv<1>(pl, in, out, B, s);
-  if (blocks < 4 * (int64_t)device_cus()) return launch_inv<2>(pl, in, out, B, s);
+  if (pl->Jh <= 32 || blocks < 4 * (int64_t)device_cus()) return launch_inv<2>(pl, in, out, B, s);
   return launch_inv<4>(pl, in, out, B, s);
 }
 
