@@ -136,9 +136,15 @@ struct MP {
 // 4.9, 5.8, 8.2 / 5.2, 6.3, 9.3; T85 L24 moist (3.6e5) 7.0, 7.6, 9.5 / 9.7, 9.9, 13.7;
 // T42 L24, 4 members (3.6e5) 5.8, 5.7, 6.2 / 6.2, 5.5, 6.1; TL255 L37 moist (4.9e6)
 // 44, 39, 42 / 83, 79, 83, 16 members (7.8e7) 996, 985, 983 / 1225, 1158, 1144, their
-// adjoints 1104, 1009, 995 / 1509, 1525, 1545.
-inline int levels_per_thread(int64_t entries) {
-  return entries <= (1 << 18) ? 1 : entries <= (1 << 25) ? 2 : 4;
+// adjoints 1104, 1009, 995 / 1509, 1525, 1545.  Without tracers the epilogue and the
+// prep's adjoint (`stencils`: mostly stencils, few plain copies) gain from four levels
+// earlier, with 2 and 4: T85 L37, 3 members (1.65e6) 14.4, 13.3 / 13.6, 12.8; TL255 L37
+// (4.9e6) 30.0, 27.1 / 27.2, 26.0; FP64 4 members (2.2e6) 23.0, 24.8 / 22.5, 23.8, TL127 L32, 8
+// members (8.4e6) 124, 116 / 116, 114; prep and the epilogue's adjoint do not (TL255 21.6,
+// 20.8 / 22.7, 22.4; 4 members 123, 125 / 144, 150).
+inline int levels_per_thread(int64_t entries, bool stencils, size_t es) {
+  const int64_t four = !stencils ? 1 << 25 : es == 4 ? 1 << 20 : 1 << 22;
+  return entries <= (1 << 18) ? 1 : entries <= four ? 2 : 4;
 }
 
 // Stencil of one thread's (r, l): the bidiagonal-in-l operators read the
@@ -513,7 +519,7 @@ const T* consts(const dino_modal* m) {
   else return m->c32;
 }
 
-MP make_mp(const dino_modal* m, int64_t E) {
+MP make_mp(const dino_modal* m) {
   MP p;
   p.R = m->R;
   p.L = m->L;
@@ -523,8 +529,8 @@ MP make_mp(const dino_modal* m, int64_t E) {
   p.lnps = m->hybrid || m->forced;
   p.forced = m->forced;
   p.RL = (int64_t)m->R * m->L;
-  p.kc = std::min(levels_per_thread(p.RL * m->K * E), m->K);
-  p.nkc = (m->K + p.kc - 1) / p.kc;
+  p.kc = m->K;
+  p.nkc = 1;
   p.a = m->radius;
   p.g = m->gravity;
   return p;
@@ -533,7 +539,10 @@ MP make_mp(const dino_modal* m, int64_t E) {
 template <typename T>
 int run(int which, const dino_modal* m, const void* a, const void* b, void* out, int64_t E,
         hipStream_t s) {
-  MP p = make_mp(m, E);
+  MP p = make_mp(m);
+  const bool stencils = m->nt == 0 && (which == 1 || which == 2);
+  p.kc = std::min(levels_per_thread(p.RL * m->K * E, stencils, sizeof(T)), m->K);
+  p.nkc = (m->K + p.kc - 1) / p.kc;
   // level chunks: as many as the grid's y extent allows for E members
   while ((int64_t)p.nkc * E > 65535) {
     p.kc *= 2;
@@ -570,7 +579,7 @@ int run(int which, const dino_modal* m, const void* a, const void* b, void* out,
 template <typename T>
 int run_winds(int mode, const dino_modal* m, const void* x0, const void* x1, void* y0, void* y1,
               int64_t B, int clip, hipStream_t s) {
-  const MP p = make_mp(m, 1);
+  const MP p = make_mp(m);
   // Fields per thread: a thread has little else to do, so four share the stencil from
   // 1e6 entries on (modes 0 and 2 with 1, 2, 4: TL159 37 fields 8.1, 6.8, 6.4 / 10.5, 7.9,
   // 7.3 us), and fewer gain half a microsecond below (T21 12 fields 3.3, 3.7, 3.9).

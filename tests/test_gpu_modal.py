@@ -14,16 +14,23 @@ pytestmark = pytest.mark.gpu
 # L13 on the two-level side of 2^25 and 174 on the four-level side (a rest of one).
 # Every member equals the member alone, a thread a level: the sums are the same.
 @pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
-@pytest.mark.parametrize('name,K,members,check', [
-    ('T21', 11, 24, range(24)), ('T21', 11, 25, range(25)),
-    ('T85', 13, 173, (0, 100, 172)), ('T85', 13, 174, (0, 100, 173))])
+# Without tracers the epilogue and the prep's adjoint change at 2^20 (FP32) and 2^22 (FP64):
+# 5 and 6, 21 and 22 members of T85 L13.
+@pytest.mark.parametrize('name,K,members,check,tracers', [
+    ('T21', 11, 24, range(24), 1), ('T21', 11, 25, range(25), 1),
+    ('T85', 13, 173, (0, 100, 172), 1), ('T85', 13, 174, (0, 100, 173), 1),
+    ('T85', 13, 5, (0, 4), 0), ('T85', 13, 6, (0, 5), 0), ('T85', 13, 21, (0, 20), 0),
+    ('T85', 13, 22, (0, 21), 0)])
 @pytest.mark.parametrize('fn', ['prep', 'prep_adjoint', 'epilogue', 'epilogue_adjoint'])
-def test_members_of_a_batch_equal_members_alone(fn, name, K, members, check, dtype, gpu_device):
+def test_members_of_a_batch_equal_members_alone(fn, name, K, members, check, tracers, dtype,
+                                                gpu_device):
   grid = getattr(sh.Grid, name)()
   R, L = grid.modal_shape
-  h = pe.modal_handle(grid, K, 1, 0, 9.8, gpu_device)
+  h = pe.modal_handle(grid, K, tracers, tracers - 1, 9.8, gpu_device)
   levels = {'state': [K, K, K, 1, K], 'prep': [K] * 6 + [1, 1, 1, K, K],
             'epilogue': [K] * 6 + [1] + [K] * 5}
+  if not tracers:
+    levels = {'state': [K, K, K, 1], 'prep': [K] * 5 + [1, 1], 'epilogue': [K] * 6 + [1]}
   groups = ('state', 'prep', 'epilogue')
   src, dst = {'prep': (0, 1), 'prep_adjoint': (1, 0), 'epilogue': (2, 0),
               'epilogue_adjoint': (0, 2)}[fn]
