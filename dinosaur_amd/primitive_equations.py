@@ -531,6 +531,7 @@ class _NodalForced(torch.autograd.Function):
       _lib.tally('held_suarez', field * E * (8 * K + 1))
     ctx.save_for_backward(nodal)
     ctx.h, ctx.forcing, ctx.members, ctx.code, ctx.groups = h, forcing, E, code, groups
+    ctx.K = K
     return out
 
   @staticmethod
@@ -549,7 +550,8 @@ class _NodalForced(torch.autograd.Function):
                  'dino_held_suarez_nodal_adjoint')
     field = g.element_size() * nodal[0].numel()
     _lib.tally('nodal_adjoint', field * (2 * nodal.shape[0] + g.shape[0]))
-    _lib.tally('held_suarez', field * (2 * nodal.shape[0] + g.shape[0]))
+    # CU, CV, HT and ln ps read, U, V, T read and written, ln ps written
+    _lib.tally('held_suarez', field * E * (9 * ctx.K + 2))
     return gin, None, None, None, None, None
 
 

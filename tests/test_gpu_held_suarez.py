@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 import torch
 
-from dinosaur_amd import held_suarez, primitive_equations as pe, time_integration as ti
+from dinosaur_amd import _lib, held_suarez, primitive_equations as pe, time_integration as ti
 from dinosaur_amd import units, workloads
 
 pytestmark = pytest.mark.gpu
@@ -116,3 +116,18 @@ def test_changed_parameters_are_used(gpu_device, name):
   for b, x, y in zip(before, run(hs), run(new)):
     assert all(p.equal(q) for p, q in zip(_leaves(x), _leaves(y)))
     assert not all(p.equal(q) for p, q in zip(_leaves(b), _leaves(x)))
+
+
+def test_work_of_the_forcing_kernels(gpu_device):
+  """Fields that the kernels read and write (8 K + 1 forward, 9 K + 2 adjoint)."""
+  K, members = 5, 2
+  eq, hs, st, coords, _ = _setup(K, members, False, torch.float32, gpu_device)
+  x = st.as_flat().flat_buffer().clone().requires_grad_(True)
+  state = pe.State.from_flat(x, (members,), K, ())
+  field = 4 * coords.horizontal.nodal_shape[0] * coords.horizontal.nodal_shape[1]
+  with _lib.work_tally() as t:
+    out = hs.fused_with(eq).explicit_terms(state).flat_buffer()
+    forward = t.families['held_suarez']['bytes']
+    out.sum().backward()
+  assert forward == field * members * (8 * K + 1)
+  assert t.families['held_suarez']['bytes'] - forward == field * members * (9 * K + 2)
