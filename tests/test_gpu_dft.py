@@ -93,3 +93,35 @@ def test_dft_matches_numpy(gpu_device, shape, dtype):
       got = out[1].double().cpu().numpy()
       assert np.linalg.norm(got - ref) <= tol * np.linalg.norm(ref), ('inverse', weighted, skew)
       assert (out[0][skew + x.numel():] == 7.0).all() and (out[0][:skew] == 7.0).all()
+
+
+# Kernels: per-tile FFT, persistent FFT (FP32), folded DFT, mixed-radix FFT, direct DFT;
+# (9, 1, 6) the direct one of short lengths.
+@pytest.mark.parametrize('dtype', [torch.float32, torch.float64])
+@pytest.mark.parametrize('shape', [(64, 22, 32), (512, 170, 256), (128, 43, 64), (67, 22, 34),
+                                   (320, 107, 160), (583, 291, 40), (9, 1, 6)])
+def test_secant_weights(gpu_device, shape, dtype):
+  """DINO_SHT_SEC_LAT: nodal values over cos(lat) after an inverse and before a forward
+  transform, and in both adjoints: one rounding of the weight and one of the product
+  more than the transform without it."""
+  I, M, J = shape
+  L = M + 1
+  plan = sh.get_plan(M, L, I, J, 'gauss', gpu_device)
+  print('[test] secant weights', shape, dtype, flush=True)
+  node = plan.nodes()[0]
+  sec = torch.as_tensor(1 / np.sqrt((1 - node) * (1 + node)), device=gpu_device)
+  tol = 8 * np.sqrt(max(I, J)) * (2.0 ** -24 if dtype == torch.float32 else 2.0 ** -53)
+  gen = torch.Generator(device=gpu_device).manual_seed(I)
+  x = torch.randn((5, I, J), generator=gen, device=gpu_device, dtype=torch.float64).to(dtype)
+  m = torch.randn((5, 2 * M - 1, L), generator=gen, device=gpu_device,
+                  dtype=torch.float64).to(dtype)
+  m = m * (torch.arange(L, device=gpu_device) >= (torch.arange(2 * M - 1, device=gpu_device)[:, None]
+                                                  + 1) // 2)
+  scaled = lambda t: (t.double() * sec).to(dtype)  # noqa: E731
+  call = lambda name, src, tail, flag: sh.sht_call(name, plan, src, tail, flag).double()  # noqa: E731
+  for name, src, tail in (('dino_sht_inverse', m, (I, J)), ('dino_sht_forward_adjoint', m, (I, J)),
+                          ('dino_sht_forward', x, (2 * M - 1, L)),
+                          ('dino_sht_inverse_adjoint', x, (2 * M - 1, L))):
+    got = call(name, src, tail, _lib.SHT_SEC_LAT)
+    ref = call(name, src, tail, 0) * sec if src is m else call(name, scaled(src), tail, 0)
+    assert (got - ref).norm() <= tol * ref.norm(), name
