@@ -46,9 +46,11 @@ constexpr int kWavesPerBlock = 8;  // waves sharing one LDS copy of the tables
 // two tiles a wave: T21 L12 (62 tiles) 5.0 / 7.2 us, TL127 L32 (2056) 15.6 / 20.1,
 // TL127 L32, 4 members (8224) 34.1 / 34.7, 8 members (16448) 60.0 / 61.3, TL255 L37,
 // 4 members (32832) 145 / 129, 16 members (131328) 539 / 474; four: 11.7, 35.0,
-// 49.1, 63.4, 139, 479.
+// 49.1, 63.4, 139, 479.  FP64: TL127 L32 16.4 / 21.4, 8 members 68.7 / 75.5, TL255 L37, 4
+// members 228 / 206, 8 members 440 / 390.
+constexpr int kMaxTilesPerWave = 2;
 inline int tiles_per_wave(int64_t tiles) {
-  return tiles <= (int64_t)8 * kWavesPerBlock * device_cus() ? 1 : 2;
+  return tiles <= (int64_t)8 * kWavesPerBlock * device_cus() ? 1 : kMaxTilesPerWave;
 }
 
 __device__ __forceinline__ doublex4 mma64(double a, double b, doublex4 c) {
@@ -462,7 +464,7 @@ static int launch_ns(bool solve, bool adjoint, bool acc, const dino_implicit* f,
   const int64_t waves = (cols + 15) / 16 * members;
   if (waves == 0) return DINO_OK;
   // column tiles and columns are indexed with 32-bit integers in the kernels
-  DINO_REQUIRE(waves + (int64_t)kWavesPerBlock * 4 < ((int64_t)1 << 31) &&
+  DINO_REQUIRE(waves + (int64_t)kWavesPerBlock * kMaxTilesPerWave < ((int64_t)1 << 31) &&
                    cols < ((int64_t)1 << 31),
                DINO_EINVAL, "implicit solve: too many columns for one launch");
   const int repeats = tiles_per_wave(waves);

@@ -580,9 +580,9 @@ template <typename T>
 int run_winds(int mode, const dino_modal* m, const void* x0, const void* x1, void* y0, void* y1,
               int64_t B, int clip, hipStream_t s) {
   const MP p = make_mp(m);
-  // Fields per thread: a thread has little else to do, so four share the stencil from
-  // 1e6 entries on (modes 0 and 2 with 1, 2, 4: TL159 37 fields 8.1, 6.8, 6.4 / 10.5, 7.9,
-  // 7.3 us), and fewer gain half a microsecond below (T21 12 fields 3.3, 3.7, 3.9).
+  // Four fields a thread share the stencil, at every size: a thread has little else to
+  // do (modes 0 and 2 with 1, 2, 4: TL159 37 fields 8.1, 6.8, 6.4 / 10.5, 7.9, 7.3 us), and
+  // where fewer are better it is by half a microsecond (T21 12 fields 3.3, 3.7, 3.9).
   int64_t per = 4;
   while ((B + per - 1) / per > 65535) per *= 2;
   const bool tiles = mode == 0 || mode == 3;  // outputs the inverse transform reads

@@ -29,6 +29,7 @@
 // (primitive_equations.py:1001-1059, 1126-1194), so one field carries their
 // sum through the forward transform instead of two.
 #include <cstring>
+#include <type_traits>
 
 #include "dino_common.h"
 
@@ -77,17 +78,19 @@ constexpr int MAXTR = 6;
 constexpr int kNodalWaves = 8;
 constexpr size_t kLdsBytes = 160 * 1024;  // of a CU
 inline int nodal_waves(int K) { return K / 2 < 1 ? 1 : K / 2 < kNodalWaves ? K / 2 : kNodalWaves; }
-// Bytes of LDS of a split block: what the column sums take of each level.
-inline size_t split_lds(int K, bool moist, size_t es) { return 64 * es * (moist ? 4 : 3) * (size_t)K; }
-// Batches the split form takes (members x columns): those of few bytes a field, the more
-// the more levels there are to share.  Whole columns / split, us: FP32 T42 L24 dry, 1
-// member (8192 columns) 29.9 / 10.8, 12 members (98304) 43.6 / 34.2, 32 (262144) 66 / 92;
-// L24 moist 98304 87 / 75, 131072 106 / 124; L12 dry 65536 19.2 / 16.9, 98304 23.0 / 25.6;
-// L5 moist 32768 14.3 / 14.1, 65536 16.4 / 17.8; L2 8192 5.3 / 5.9.  FP64 L24 dry 8192
-// 35 / 12.8, 49152 44.7 / 36.6, 65536 46.3 / 46.4, 98304 51 / 66; L12 32768 21.7 / 17.8, 49152
-// 23.5 / 25.2.  Beyond 160 KiB of LDS (FP32 above 160 moist levels): whole columns.
+// Bytes of LDS of a split block: what the column sums take of each level, and the sums.
+inline size_t split_lds(int K, bool moist, size_t es) {
+  return 64 * es * ((moist ? 4 : 3) * (size_t)K + 3);
+}
+// Batches the split form takes (columns of all members), more the more levels there are
+// to share.  Whole columns / split, us: FP32 T42 L24 dry, 1 member (8192 columns) 30.0 /
+// 10.5, 12 members (98304) 43.4 / 32.0, 16 (131072) 44.8 / 39.6, 32 (262144) 70 / 82; L24
+// moist 98304 75 / 57, 262144 166 / 184; L12 dry 49152 17.9 / 14.3, 98304 23.1 / 26.7; L5 moist
+// 32768 14.3 / 13.5, 65536 16.3 / 16.6; L2 8192 5.3 / 5.9.  FP64 L24 dry 8192 35.3 / 11.9, 98304
+// 51.5 / 47.3; moist 98304 137 / 129, 131072 161 / 168; L12 dry 49152 23.6 / 18.9, 65536 24.3 /
+// 27.3.  Beyond 160 KiB of LDS (FP32 above 159 moist levels, FP64 above 79): whole columns.
 inline bool nodal_split(int64_t columns, int K, bool moist, size_t es) {
-  return K >= 4 && columns * (int64_t)es <= (int64_t)24576 * (K < 16 ? K : 16) &&
+  return K >= 4 && columns <= (int64_t)4096 * (K < 24 ? K : 24) &&
          split_lds(K, moist, es) <= kLdsBytes;
 }
 
@@ -168,17 +171,20 @@ __device__ __forceinline__ T rounded_sum(T a, T b) {
 // Pass A forms the column totals, pass B streams the levels with a (k, k + 1)
 // window.  A thread walks all levels of its column, or (SPLIT) a block owns 64
 // columns and each of its waves a contiguous share of the levels: what the sums
-// take of each level meets in LDS, every wave sums it in level order (totals, and
-// prefixes up to its first level) and forms the flux through its top interface from
-// the level above.  Both forms add the same terms in the same order, so a member's
-// values do not depend on the batch.  Whole columns stream every field once, in order,
-// at the copy rate, but a grid of a few thousand columns is then a few dozen waves in a
-// long chain (nodal_split: both sides measured).
+// take of each level meets in LDS, each sum runs in level order in one wave, and a
+// wave starts from the prefixes at its first level and the flux through its top
+// interface, formed from the level above.  Both forms add the same terms in the same
+// order, so a member's values do not depend on the batch (two barriers and a chain of K
+// sums: 0.5 us of a launch).  Whole columns stream every field once, in order, at the
+// copy rate, but a grid of a few thousand columns is then a few dozen waves in a long
+// chain (nodal_split: both sides measured).
 template <typename T, bool SPLIT>
 __global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_kernel(
     const T* __restrict__ in, T* __restrict__ out, const T* __restrict__ cst, Groups g,
     Params p) {
-  const int lane = threadIdx.x, wave = SPLIT ? (int)threadIdx.y : 0;
+  // a wave is one threadIdx.y: its levels are scalars
+  const int lane = threadIdx.x;
+  const int wave = SPLIT ? __builtin_amdgcn_readfirstlane((int)threadIdx.y) : 0;
   const int G = SPLIT ? (int)blockDim.y : 1;
   const int64_t col = (int64_t)blockIdx.x * blockDim.x + lane;
   const int64_t e = blockIdx.y;
@@ -221,29 +227,76 @@ __global__ __launch_bounds__(SPLIT ? 64 * kNodalWaves : 256) void nodal_forward_
   };
   if constexpr (SPLIT) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    // what the sums take of each level: w of the totals, w of the prefixes (they
-    // round differently, see wind_sum), d, td
-    T* const lev = reinterpret_cast<T*>(smem_raw) + lane;
-    const int P = 64 * K;
-#pragma unroll 4
-    for (int k = k0; k < k1; ++k) {
-      const T u = *I_(g.u, K, k), v = *I_(g.v, K, k);
-      lev[64 * k] = wind_sum(u, gx, v, gy);
-      lev[64 * k + P] = wind_sum(v, gy, u, gx);
-      lev[64 * k + 2 * P] = *I_(g.d, K, k);
-      if (moist) lev[64 * k + 3 * P] = moist_term(k);
-    }
-    __syncthreads();
-    // the totals, and the prefixes up to this wave's first level
-    for (int k = 0; k < K; ++k) {
-      const T d = lev[64 * k + 2 * P];
-      add_level(k, lev[64 * k], d, &TE, &TF);
-      if (k < k0) add_level(k, lev[64 * k + P], d, &PE, &PF);
-      if (moist) {
-        if (k == k0) GP = GT;
-        if (k >= 1) GT = fma(cst[o.gp + k], lev[64 * k + 3 * P], GT);
+    // what the sums take of each level: w of the totals, w of the prefixes (they round
+    // differently, see wind_sum), d, td
+    T* const wt = reinterpret_cast<T*>(smem_raw) + lane;
+    T *const wp = wt + 64 * K, *const dl = wp + 64 * K, *const tl = dl + 64 * K;
+    // four levels' loads in flight (past the wave's last level: that one again)
+    for (int kb = k0; kb < k1; kb += 4) {
+      T u[4], v[4], d[4], td[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = kb + q < k1 ? kb + q : k1 - 1;
+        u[q] = *I_(g.u, K, k);
+        v[q] = *I_(g.v, K, k);
+        d[q] = *I_(g.d, K, k);
+        td[q] = moist ? moist_term(k) : (T)0;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = kb + q;
+        if (k >= k1) break;
+        wt[64 * k] = wind_sum(u[q], gx, v[q], gy);
+        wp[64 * k] = wind_sum(v[q], gy, u[q], gx);
+        dl[64 * k] = d[q];
+        if (moist) tl[64 * k] = td[q];
       }
     }
+    __syncthreads();
+    // Sums in level order: the totals in the first wave, whose prefixes are empty, the
+    // prefixes up to its first level in each other one; eight levels at a time, so that
+    // their reads are in flight together.
+    const int n = wave == 0 ? K : k0;
+    const T* const wl = wave == 0 ? wt : wp;
+    auto add8 = [&](auto whole, int kb) {
+      T a[8], d[8], h[8], y[8], r[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int k = whole.value || kb + q < n ? kb + q : n - 1;
+        a[q] = wl[64 * k];
+        d[q] = dl[64 * k];
+        h[q] = cst[o.dsig + k];
+        if (moist) {
+          y[q] = tl[64 * k];
+          r[q] = cst[o.gp + k];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const bool in = whole.value || kb + q < n;
+        const T e = fma(a[q] * s, h[q], PE), f = fma(fma(a[q], s, d[q]), h[q], PF);
+        PE = in ? e : PE;
+        PF = in ? f : PF;
+        if (moist) {
+          const T sum = fma(r[q], y[q], GP);
+          GP = in && kb + q >= 1 ? sum : GP;
+        }
+      }
+    };
+    int kb = 0;
+    for (; kb + 8 <= n; kb += 8) add8(std::true_type{}, kb);
+    if (kb < n) add8(std::false_type{}, kb);
+    T* const total = dl + 64 * K * (moist ? 2 : 1);
+    if (wave == 0) {
+      total[0] = PE;
+      total[64] = PF;
+      total[128] = GP;
+      PE = PF = GP = 0;
+    }
+    __syncthreads();
+    TE = total[0];
+    TF = total[64];
+    GT = total[128];
   } else {
     for (int k = 0; k < K; ++k) {
       const T u = *I_(g.u, K, k), v = *I_(g.v, K, k);

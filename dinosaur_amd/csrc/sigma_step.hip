@@ -7,8 +7,8 @@
 // same order, on the caller's stream and workspace, so results are bitwise the
 // same.  It exists for the small grids, where a step's 31 launches of 4-10 us
 // each cost 18-20 us apiece from Python: T21 L12, one member, a SIL3 step with
-// its filter, 641 us through the separate calls and 172 in one; T42 L24 explicit terms
-// 141 and 71 us.
+// its filter, 641 us through the separate calls and 227 in one, with the same kernels;
+// T42 L24 explicit terms 141 and 77 us.
 #include <algorithm>
 #include <vector>
 

@@ -20,14 +20,14 @@ def _ragged():
 
 
 # Levels: one wave (1 to 3), an uneven share (5, 17, 37), the model's (12);
-# 3 and 4 members of T42 L8 lie on both sides of the batches where the whole-column
-# kernel takes over (FP64), 12 and 13 members of two levels both beyond.
+# 4 and 5 members of T42 L8 lie on both sides of the batches where the whole-column
+# kernel takes over, 12 and 13 members of two levels both beyond.
 @pytest.mark.parametrize('grid,K,members,moist,tref_varies', [
     (_ragged, 1, 1, False, False), (_ragged, 2, 3, True, True), (_ragged, 3, 1, False, True),
     (_ragged, 5, 2, True, False), (_ragged, 17, 1, True, True), (_ragged, 37, 2, False, True),
     (sh.Grid.T21, 12, 1, True, True), (sh.Grid.T42, 2, 12, True, True),
-    (sh.Grid.T42, 2, 13, True, True), (sh.Grid.T42, 8, 3, True, True),
-    (sh.Grid.T42, 8, 4, True, True)])
+    (sh.Grid.T42, 2, 13, True, True), (sh.Grid.T42, 8, 4, True, True),
+    (sh.Grid.T42, 8, 5, True, True)])
 def test_split_and_whole_columns_match_unfused(grid, K, members, moist, tref_varies, gpu_device):
   grid = grid()
   coords = coordinate_systems.CoordinateSystem(
@@ -65,7 +65,7 @@ def test_split_and_whole_columns_match_unfused(grid, K, members, moist, tref_var
 @pytest.mark.parametrize('K,moist,tref_varies', [(1, False, False), (2, True, True),
                                                  (3, False, True), (5, True, False),
                                                  (8, False, True), (17, True, True),
-                                                 (37, True, True)])
+                                                 (37, True, True), (64, True, False)])
 def test_member_in_a_batch_equals_the_member_alone(gpu_device, K, moist, tref_varies, dtype):
   print('[test] nodal member alone', K, moist, dtype, flush=True)
   members = 600
