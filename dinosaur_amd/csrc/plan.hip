@@ -147,6 +147,9 @@ __global__ void twiddle_kernel(int n, double* tw64, float* tw32) {
 
 __global__ void latitude_weights_kernel(int I, int J, int stride, const double* x,
                                         const double* w, double* q64, float* q32) {
+// as Grid.cos_lat rounds it: without a fused product, whose cosine differs near the
+// poles by more than the transforms' rounding
+#pragma clang fp contract(off)
   int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= J) return;
   const double pi = 3.14159265358979323846;
