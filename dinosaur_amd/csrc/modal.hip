@@ -460,6 +460,10 @@ __global__ __launch_bounds__(256) void epilogue_adjoint_kernel(const T* __restri
 //   0: (vorticity, divergence) -> (u cos, v cos), read by the inverse transform
 //   1: its adjoint             2: (u, v) / cos -> (vorticity, divergence)
 //   3: its adjoint, read by the inverse transform
+// FP64 coefficients and arithmetic for FP32 fields too, one rounding of each result:
+// the polar winds amplify what is lost here (u against float64, T85, 16 levels: 5.6e-7
+// with FP32 arithmetic, 5.2e-7 with FP32 fields on FP64 coefficients, 4.6e-7 now, as from
+// exactly rounded modal winds).  It costs 7 us of 74 a launch at TL255, 222 fields.
 // One pass over both fields instead of about 20 elementwise tensor operations
 // of the composed operators; bound by launches at common sizes (37 levels of
 // TL159: 3.8 MB in and out of each).
@@ -467,7 +471,7 @@ template <typename T, int MODE>
 __global__ __launch_bounds__(256) void winds_kernel(const T* __restrict__ x0,
                                                     const T* __restrict__ x1,
                                                     T* __restrict__ y0, T* __restrict__ y1,
-                                                    const T* __restrict__ cst,
+                                                    const double* __restrict__ cst,
                                                     const int* __restrict__ tile_pos,
                                                     int64_t n_pos, int64_t B, int per, int clip,
                                                     MP p) {
@@ -478,38 +482,39 @@ __global__ __launch_bounds__(256) void winds_kernel(const T* __restrict__ x0,
   const int64_t pos = tile_pos ? tile_pos[q] : q;
   const int r = (int)(pos / p.L), l = (int)(pos % p.L);
   const MOff o = moff(p.R, p.L);
-  Stencil<T> S(cst, o, p.R, p.L, r, l);
-  const T inva = (T)(1.0 / p.a);
-  const T il = cst[o.il + l];
-  const T mk = clip ? cst[o.mask + l] : (T)1;
-  const T mk_m = clip ? cst[o.mask + S.lm] : (T)1, mk_p = clip ? cst[o.mask + S.lp] : (T)1;
+  const Stencil<double> S(cst, o, p.R, p.L, r, l);
+  const double inva = 1.0 / p.a;
+  const double mk = clip ? cst[o.mask + l] : 1;
+  const double mk_m = clip ? cst[o.mask + S.lm] : 1, mk_p = clip ? cst[o.mask + S.lp] : 1;
+  // y0 = lon x1 - (up x0[l + 1] + dn x0[l - 1]), y1 = lon x0 + (up x1[l + 1] + dn x1[l - 1]);
+  // the adjoints (1, 3) have the transposed stencil of the clipped cotangent
+  double lon, up, dn;
+  if (MODE == 0) {
+    lon = S.jr * cst[o.il + l] * inva * mk;
+    up = S.up_p * S.il_p * inva * mk;
+    dn = S.dn_m * S.il_m * inva * mk;
+  } else if (MODE == 2) {
+    lon = S.jr * inva * mk;
+    up = S.up2_p * inva * mk;
+    dn = S.dn2_m * inva * mk;
+  } else {
+    const double f = MODE == 1 ? cst[o.il + l] * inva : inva;
+    lon = -S.jr * f * mk;
+    up = (MODE == 1 ? S.dn_l : S.dn2_l) * f * mk_p;
+    dn = (MODE == 1 ? S.up_l : S.up2_l) * f * mk_m;
+  }
   const bool tri = l < ((r + 1) >> 1);  // zero, and what it would read may be unwritten
-  // transposed stencils of the clipped cotangent
-  auto dlon_k = [&](const T* y) -> T { return S.jr * y[S.prow + l] * mk; };
-  auto up_down = [&](const T* y, T up, T dn) -> T {
-    const T a = up * (y[S.row + S.lm] * mk_m), b = dn * (y[S.row + S.lp] * mk_p);
-    return (S.hm ? a : (T)0) + (S.hp ? b : (T)0);
-  };
   for (int64_t b = (int64_t)by * per; b < B && b < (int64_t)(by + 1) * per; ++b) {
     const T *u = x0 + b * p.RL, *v = x1 + b * p.RL;
-    T s = 0, t = 0;
+    double s = 0, t = 0;
     if (!tri) {
-      if (MODE == 0) {
-        s = (S.dlon(v) * il - S.cldl_il(u)) * inva * mk;
-        t = (S.cldl_il(v) + S.dlon(u) * il) * inva * mk;
-      } else if (MODE == 1) {
-        s = il * ((-up_down(u, S.up_l, S.dn_l) - dlon_k(v)) * inva);
-        t = il * ((-dlon_k(u) + up_down(v, S.up_l, S.dn_l)) * inva);
-      } else if (MODE == 2) {
-        s = (S.dlon(v) - S.sdlc(u)) * inva * mk;
-        t = (S.dlon(u) + S.sdlc(v)) * inva * mk;
-      } else {
-        s = (-up_down(u, S.up2_l, S.dn2_l) - dlon_k(v)) * inva;
-        t = (-dlon_k(u) + up_down(v, S.up2_l, S.dn2_l)) * inva;
-      }
+      const double up_u = up * u[S.row + S.lp], dn_u = dn * u[S.row + S.lm];
+      const double up_v = up * v[S.row + S.lp], dn_v = dn * v[S.row + S.lm];
+      s = lon * v[S.prow + l] - ((S.hp ? up_u : 0) + (S.hm ? dn_u : 0));
+      t = lon * u[S.prow + l] + ((S.hp ? up_v : 0) + (S.hm ? dn_v : 0));
     }
-    y0[b * p.RL + pos] = s;
-    y1[b * p.RL + pos] = t;
+    y0[b * p.RL + pos] = (T)s;
+    y1[b * p.RL + pos] = (T)t;
   }
 }
 
@@ -580,16 +585,17 @@ template <typename T>
 int run_winds(int mode, const dino_modal* m, const void* x0, const void* x1, void* y0, void* y1,
               int64_t B, int clip, hipStream_t s) {
   const MP p = make_mp(m);
-  // Four fields a thread share the stencil, at every size: a thread has little else to
-  // do (modes 0 and 2 with 1, 2, 4: TL159 37 fields 8.1, 6.8, 6.4 / 10.5, 7.9, 7.3 us), and
-  // where fewer are better it is by half a microsecond (T21 12 fields 3.3, 3.7, 3.9).
-  int64_t per = 4;
+  // Fields a thread: they share the stencil's coefficients.  Modes 0 and 2 with 2, 4, 8,
+  // us: T21 12 fields 3.8, 4.3, 5.1 / 3.6, 4.1, 4.9; TL159 37 (1.9e6 entries) 8.5, 8.0, 8.0 /
+  // 9.5, 8.8, 8.7; TL255 37 (4.9e6) 15.3, 13.5, 12.4 / 18.2, 15.5, 15.3, 222 101, 86, 81 / 130,
+  // 113, 110.
+  int64_t per = p.RL * B > (1 << 21) ? 8 : 4;
   while ((B + per - 1) / per > 65535) per *= 2;
   const bool tiles = mode == 0 || mode == 3;  // outputs the inverse transform reads
   const int64_t n = tiles ? m->n_tile_pos : p.RL;
   const dim3 grid((unsigned)((n + 255) / 256), (unsigned)((B + per - 1) / per));
   const int* tp = tiles ? m->tile_pos : nullptr;
-  const T* c = consts<T>(m);
+  const double* const c = m->c64;
 #define WINDS(MODE)                                                                         \
   winds_kernel<T, MODE><<<grid, 256, 0, s>>>((const T*)x0, (const T*)x1, (T*)y0, (T*)y1, c, tp, \
                                              n, B, (int)per, clip, p)

@@ -129,3 +129,25 @@ def test_equal_grids_share_one_handle(gpu_device):
 
   first = handle()
   assert handle() is first and handle(radius=2.0) is not first
+
+
+# 12 and 200 fields: 4 and 8 a thread
+@pytest.mark.parametrize('fields', [12, 200])
+def test_modal_winds_are_rounded_once(gpu_device, fields):
+  """FP32 fields: each result is the FP64 one rounded, whose error the polar winds
+  amplify no further."""
+  grid = sh.Grid.T85()
+  gen = torch.Generator(device=gpu_device).manual_seed(3)
+  mask = torch.as_tensor(grid.mask, device=gpu_device)
+  a, b = (torch.randn((fields,) + grid.modal_shape, generator=gen, device=gpu_device) * mask
+          for _ in range(2))
+  handle = sh._winds_handle(grid, a, b, grid.modal_shape)
+  a64, b64 = a.double(), b.double()
+  exact = {0: sh.get_cos_lat_vector(a64, b64, grid),
+           2: (grid.curl_cos_lat((a64, b64)), grid.div_cos_lat((a64, b64)))}
+  for mode, refs in exact.items():
+    got = sh._Winds.apply(a, b, handle, mode, True).double()
+    for x, ref in zip((got[:fields], got[fields:]), refs):
+      err = torch.where(mask, x - ref, 0.0).abs()  # below the triangle: not all written
+      # half an ulp, and the FP64 terms' own rounding
+      assert (err <= 2.0 ** -24 * ref.abs() + 1e-14 * ref.abs().max()).all(), mode
