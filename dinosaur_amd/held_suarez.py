@@ -45,10 +45,11 @@ class HeldSuarezForcingSigma(time_integration.ExplicitODE):
                                            * np.cos(self.lat) ** 4)
 
   def _parameters(self):
-    """What the constants below are made of, as a cache key."""
-    arrays = (self.sigma, self.reference_temperature, self.lat[0])
+    """What the constants below are made of, as a cache key.  Constants of former
+    values stay for the object's life: captured graphs may read them."""
     return (float(self.sigma_b), float(self.kf), float(self.ka), float(self.ks),
-            *(np.asarray(a, np.float64).tobytes() for a in arrays))
+            np.asarray(self.sigma).tobytes(), np.asarray(self.reference_temperature).tobytes(),
+            np.asarray(self.lat[0]).tobytes())
 
   def _c(self, name, like):
     key = (name, like.device, like.dtype, self._parameters())
